@@ -25,6 +25,7 @@ CSRC = os.path.join(PKG, "csrc")
 # The GEMM's tiles are spread over several sources (gemm_tiles.h), listed
 # first: their device code takes longest to generate.
 HIP_SOURCES = ["hip/gemm_tiles_pipe_a.hip", "hip/gemm_tiles_pipe_b.hip",
+               "hip/gemm_tiles_pipe_c.hip", "hip/gemm_tiles_single_mid.hip",
                "hip/gemm_tiles_single.hip", "hip/gemm_tiles_mid.hip", "hip/gemm_tiles_small.hip",
                "hip/gemm_tiles_w8_large.hip", "hip/gemm_tiles_w8.hip",
                "hip/gemm_tiles_w8_small.hip", "hip/gemm.hip", "hip/panel_gemm.hip", "hip/skinny_gemm.hip", "hip/attention.hip", "hip/rowops.hip",

@@ -73,11 +73,12 @@ hipError_t Reduce(const GemmParams &p, const float *part, int splits, hipStream_
 template <int BM, int BN, int BK, int ST, int WM, int WN, bool SPLIT>
 hipError_t Launch(const GemmParams &p, hipStream_t stream) {
   // fp8 weights: the ring's stages when their rows go through LDS, else two
-  // (fragments from global memory).
+  // (fragments from global memory).  bf16 weights over BK = 64: the
+  // double-buffered loop.
   if (p.W8)
     return LaunchW<BM, BN, BK, W8InLds<BM, BN, BK, WM, WN, SPLIT>() ? ST : 2, WM, WN, SPLIT,
                    true>(p, stream);
-  return LaunchW<BM, BN, BK, ST, WM, WN, SPLIT, false>(p, stream);
+  return LaunchW<BM, BN, BK, ST, WM, WN, SPLIT, false, false, BK == 64>(p, stream);
 }
 
 bool Aligned(const void *ptr, std::uintptr_t bytes) {
@@ -87,11 +88,7 @@ bool Aligned(const void *ptr, std::uintptr_t bytes) {
 }  // namespace
 
 // Rows from which the tile rules for large problems apply (below them,
-// 64 x 64 tiles over the whole K or split-K).  From 1536 rows (24
-// positions) Q|K|V takes 256 x 128 split tiles instead of 1176-1519
-// whole-K 64 x 64 ones: forward at batch 24 2.47 -> 2.41 ms, 28 2.60 ->
-// 2.50, 31 2.84 -> 2.56; from 1024 rows it was slower (batch 16 2.07 ->
-// 2.34).
+// 64 x 64 tiles over the whole K or split-K).
 constexpr int kLargeRows = 1536;
 
 // 256 x 256 tiles where they fill whole rounds of 256 workgroups (bf16
@@ -101,51 +98,251 @@ bool GemmWholeRoundTiles(const GemmParams &p) {
   return p.M >= kLargeRows && p.N >= 128 && p.k_splits == 1 && big_tiles % 256 == 0 && !p.A8;
 }
 
+// (Split precision: two 128 x 256 tiles per CU.)
+bool GemmFillsCus(const GemmParams &p) {
+  const long wide = static_cast<long>((p.M + 127) / 128) * ((p.N + 255) / 256);
+  return GemmWholeRoundTiles(p) || (p.A_lo && !p.W8 && p.M >= kLargeRows && wide >= 512);
+}
+
 namespace {
 
-// The instances that compile a folded LayerNorm's epilogue, and the one a
-// GEMM with a folded LayerNorm runs on (the tiles the same shapes take
-// without it, where those are among them): split precision (bf16 hi + lo
-// activations, or the BF16X2_FP8LO codes), bf16 weights, one K slice.
-enum class LnTile { kNone, kLo8, k256, k256Beside, k256x128, k64, k64x64, kSplitK };
+// The tiles of the GEMMs with bf16 weights from kLargeRows rows on.  Those of
+// split precision compile a folded LayerNorm's epilogue.
+enum class Tile {
+  kNone,
+  kLo8,      // 256 x 256, BF16X2_FP8LO
+  k256,      // 256 x 256, three stages of 48 KiB (one workgroup per CU)
+  k256Two,   // 256 x 256, two stages (beside the smolgen chain)
+  k128x256,  // 128 x 256, eight waves, three stages of 32 KiB
+  kWide,     // 128 x 256, four waves, two stages of 32 KiB (beside the chain)
+  k128,      // 128 x 128 over BK = 64, three stages of 48 KiB
+  k64x128,   // 64 x 128 over BK = 64, four stages of 32 KiB
+  k64,       // 64 x 64 over BK = 64, two stages of 24 KiB (three per CU)
+  kNarrow,   // 64 x 64 over BK = 32, two stages (narrow N, beside the chain)
+  kSplitK,   // split over K, the reduce kernel applying the LayerNorm
+  // Single bf16.
+  kOne256,      // 256 x 256, four stages of 32 KiB
+  kOneSlim,     // 256 x 128, three stages of 24 KiB (beside the chain)
+  kOne256x128,  // 256 x 128 over BK = 64, three stages of 48 KiB
+  kOne128,      // 128 x 128 over BK = 64, four stages of 32 KiB
+  kOne128Two,   // 128 x 128 over BK = 64, two stages (two per CU)
+  kOne64x128,   // 64 x 128 over BK = 64, three stages of 24 KiB (two per CU)
+  kOne64,       // 64 x 64 over BK = 64, three stages of 16 KiB (three per CU)
+};
 
-LnTile LnFoldTile(const GemmParams &p) {
+// Time of a launch, in microseconds as measured on MI355X: 3 for the launch,
+// and per round of `slots` workgroups start + (per_k + fill_k * f) * K / 1024
+// with f the share of the slots the round fills (fewer busy CUs clock higher
+// and share less bandwidth); a residual epilogue adds resid, an activation
+// act (nothing where a CU's other workgroups run meanwhile).  Fitted to
+// isolated launches at the BT4 widths and 1536 to 19200 rows; the model is
+// within 10 % of most of them and orders the tiles as measured, e.g. (split)
+// 2048 rows out-projection 12.6 us on 64 x 128, 16.5 on 128 x 128, 27.9 on
+// 128 x 256; 4096 rows 19.1 on 128 x 128, 21.0 on 64 x 128; 16384 rows 67.6
+// on 256 x 256, 80.7 on 128 x 128; FFN1 there 108.6 on 128 x 256 against
+// 119.6 on 256 x 256 (1.5 rounds).  Single bf16, out-projection at 4096 rows:
+// 14.7 on 128 x 128 (20.0-23.5 on the tiles it took before).
+struct TileTime {
+  Tile tile;
+  int bm, bn, slots;
+  float start, resid, act, per_k, fill_k;
+};
+constexpr TileTime kOneTimes[] = {
+    {Tile::kOne256, 256, 256, 256, 6.f, 7.f, 5.f, 18.f, 10.f},
+    {Tile::kOneSlim, 256, 128, 256, 6.5f, 3.f, 0.f, 10.5f, 4.5f},
+    {Tile::kOne256x128, 256, 128, 256, 5.f, 2.f, 2.5f, 9.6f, 5.4f},
+    {Tile::kOne128, 128, 128, 256, 2.f, 0.5f, 1.f, 6.f, 3.f},
+    {Tile::kOne128Two, 128, 128, 512, 2.f, 0.5f, 0.f, 10.5f, 11.f},
+    {Tile::kOne64x128, 64, 128, 512, 1.5f, 0.5f, 0.f, 1.6f, 10.f},
+    {Tile::kOne64, 64, 64, 768, 1.5f, 0.5f, 0.f, 2.1f, 6.4f},
+};
+constexpr TileTime kTileTimes[] = {
+    {Tile::k256, 256, 256, 256, 6.f, 9.f, 5.f, 29.f, 20.f},
+    {Tile::k128x256, 128, 256, 256, 3.f, 3.f, 2.f, 19.f, 8.5f},
+    {Tile::k128, 128, 128, 256, 2.5f, 1.5f, 1.f, 9.5f, 5.f},
+    {Tile::k64x128, 64, 128, 256, 1.5f, 1.f, 0.5f, 5.8f, 2.5f},
+    {Tile::k64, 64, 64, 768, 2.f, 1.f, 0.f, 6.f, 6.5f},
+};
+
+float LaunchTime(const TileTime &t, int M, const GemmParams &p) {
+  const long tiles = static_cast<long>((M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn);
+  const float k = p.K / 1024.f;
+  const float start = t.start + (p.out_mode == GEMM_OUT_RESID_F32 ? t.resid : 0.f) +
+                      (p.act != ACT_NONE ? t.act : 0.f);
+  const long full = tiles / t.slots, rem = tiles % t.slots;
+  float us = 3.f + full * (start + (t.per_k + t.fill_k) * k);
+  if (rem)
+    us += start + (t.per_k + t.fill_k * rem / t.slots) * k;
+  return us;
+}
+
+// The fastest tile by that model for M rows of p; a folded LayerNorm takes
+// whole tiles, on the residual side of kLnStatCols columns at least.
+Tile BestTile(const GemmParams &p, int M, float *us) {
+  const bool ln_res = p.out_gamma || p.res_stats;
+  Tile best = Tile::kNone;
+  *us = 0.f;
+  const auto consider = [&](const TileTime &t) {
+    if (((p.fold_c || ln_res) && p.N % t.bn) || (ln_res && t.bn < kLnStatCols))
+      return;
+    const float c = LaunchTime(t, M, p);
+    if (best == Tile::kNone || c < *us) {
+      best = t.tile;
+      *us = c;
+    }
+  };
+  if (p.A_lo)
+    for (const TileTime &t : kTileTimes)
+      consider(t);
+  else
+    for (const TileTime &t : kOneTimes)
+      consider(t);
+  return best;
+}
+
+// Rows of p to run on whole rounds of 256 x 256 tiles, the rest following as
+// a launch of its own on smaller ones (0: one launch).  A last round that is
+// nearly empty costs as much as a full one: out-projection at 19200 rows
+// (300 tiles of 256 x 256) 129 us on them, 100 on 128 x 128, 67 + 20 split.
+int RowsFirst(const GemmParams &p) {
+  if (p.N % 256 || p.beside_chain || p.M < kLargeRows)
+    return 0;
+  const TileTime &whole = p.A_lo ? kTileTimes[0] : kOneTimes[0];
+  const int nbn = p.N / 256, nbm = p.M / 256;
+  const long rounds = static_cast<long>(nbm) * nbn / 256;
+  if (rounds < 1)
+    return 0;
+  const int rows = static_cast<int>(rounds * 256 / nbn) * 256;
+  if (rows >= p.M)
+    return 0;
+  float one, rest;
+  BestTile(p, p.M, &one);
+  BestTile(p, p.M - rows, &rest);
+  return LaunchTime(whole, rows, p) + rest < 0.97f * one ? rows : 0;
+}
+
+// The tile of a large GEMM with bf16 weights, or of one with a folded
+// LayerNorm (kNone: none of these).
+Tile LargeTile(const GemmParams &p) {
   const bool res = p.out_mode == GEMM_OUT_RESID_F32;
-  if ((!p.A_lo && !p.A_lo8) || p.W8 || p.A8 || p.k_splits != 1 || p.K % 64)
-    return LnTile::kNone;
-  if (!res && p.out_mode != GEMM_OUT_BF16)
-    return LnTile::kNone;
-  // Whole rounds of 256-wide whole tiles.
+  const bool ln = p.fold_c || p.out_gamma || p.res_stats;
+  if (p.W8 || p.A8 || p.k_splits != 1 || p.K % 64)
+    return Tile::kNone;
   if (p.A_lo8)
-    return p.N % 256 == 0 ? LnTile::kLo8 : LnTile::kNone;
-  if (p.N % 256 == 0 && GemmWholeRoundTiles(p))
-    return p.beside_chain && !res ? LnTile::k256Beside : LnTile::k256;
-  // Fewer 128 x 128 tiles than CUs (24-62 positions at the BT4 widths): the
-  // 64 x 64 tiles over the whole K that these shapes take without the fold.
-  // Consumers up to 2048 wide also up to two rounds of them (FFN1 at 43-62
-  // positions, 128 x 128 tiles without the fold; on 256 x 128 ones with it
-  // the forward was 3.4 % slower at batch 48, 0.5 % at 56).
-  const long tiles128 = static_cast<long>((p.M + 127) / 128) * ((p.N + 127) / 128);
-  if (p.M >= kLargeRows && p.N >= 128 && p.N % 64 == 0 &&
-      (tiles128 < 256 || (!res && p.N <= 2048 && tiles128 < 512)))
-    return LnTile::k64x64;
-  if (res)
-    return LnTile::kNone;
-  // Consumers: the small-LDS 64 x 64 tiles beside Q|K|V (any width); narrow
-  // ones (the smolgen compression at 24-62 positions) split over K where
-  // the launcher splits them (the split GEMM sums x o gamma and the reduce
-  // kernel applies the LayerNorm before the bias), else on those 64 x 64
-  // tiles; else 256 x 128 pipelined tiles.
-  if (p.small_lds)
-    return LnTile::k64;
-  if (p.N < 128)
-    return GemmAutoSplits(p) > 1 ? LnTile::kSplitK : LnTile::k64;
-  return p.N % 128 == 0 ? LnTile::k256x128 : LnTile::kNone;
+    return !ln || p.N % 256 == 0 ? Tile::kLo8 : Tile::kNone;
+  if (!p.A_lo) {
+    if (ln || p.M < kLargeRows || p.N < 128)
+      return Tile::kNone;
+    if (p.beside_chain)
+      return GemmWholeRoundTiles(p) ? Tile::kOne256 : Tile::kOneSlim;
+    float us;
+    return BestTile(p, p.M, &us);
+  }
+  if (p.N < 128) {
+    // Narrow consumers (the smolgen compression): split over K where the
+    // launcher splits them (the split GEMM sums x o gamma and the reduce
+    // kernel applies the LayerNorm before the bias).
+    if (!ln || res)
+      return Tile::kNone;
+    return !p.small_lds && GemmAutoSplits(p) > 1 ? Tile::kSplitK : Tile::kNarrow;
+  }
+  if (p.M < kLargeRows)
+    return Tile::kNone;
+  if (p.beside_chain && !res) {
+    // Q|K|V beside the smolgen chain: two-stage tiles, so that the chain's
+    // run on the same CUs.  Forward with 128 x 256 four-wave tiles against
+    // 256 x 128 ones: batch 24 and 32 equal, 64 3155 -> 3038 us, 128 5586 ->
+    // 5464, 200 8594 -> 8357; on 128 x 128 tiles (144 KiB) 32 was 4 % slower,
+    // 64 4 %, 200 4 %.
+    if (GemmWholeRoundTiles(p) && p.N % 256 == 0)
+      return Tile::k256Two;
+    return !ln || p.N % 256 == 0 ? Tile::kWide : Tile::kNone;
+  }
+  float us;
+  return BestTile(p, p.M, &us);
+}
+
+// Rows first .. first + rows - 1 of p.
+GemmParams RowRange(const GemmParams &p, int first, int rows) {
+  GemmParams q = p;
+  const size_t r = first;
+  const auto bf16 = [](const std::uint16_t *x, size_t off) { return x ? x + off : nullptr; };
+  const bool f32 = p.out_mode != GEMM_OUT_BF16 && !p.out_gamma;
+  const auto out = [&](void *c, int ld) -> void * {
+    return c ? static_cast<char *>(c) + r * ld * (f32 ? 4 : 2) : nullptr;
+  };
+  q.M = rows;
+  q.A = bf16(p.A, r * p.lda);
+  q.A_lo = bf16(p.A_lo, r * p.lda);
+  q.C = out(p.C, p.ldc);
+  q.C_lo = out(p.C_lo, p.ldc);
+  q.C2 = out(p.C2, p.ldc2);
+  q.C2_lo = out(p.C2_lo, p.ldc2);
+  q.resid = p.resid ? p.resid + r * p.ldr : nullptr;
+  q.resid16 = bf16(p.resid16, r * p.ldr);
+  q.resid16_lo = bf16(p.resid16_lo, r * p.ldr);
+  q.C_lo8 = p.C_lo8 ? p.C_lo8 + r * p.ldc8 : nullptr;
+  const size_t stats = p.ln_width ? r * (p.ln_width / kLnStatCols) * 2 : 0;
+  q.ln_stats = p.ln_stats ? p.ln_stats + stats : nullptr;
+  q.res_stats = p.res_stats ? p.res_stats + stats : nullptr;
+  q.out_stats = p.out_stats ? p.out_stats + stats : nullptr;
+  return q;
+}
+
+hipError_t LaunchTile(Tile t, const GemmParams &p, hipStream_t stream) {
+  switch (t) {
+  case Tile::kLo8:
+    return LaunchW<256, 256, 32, 4, 4, 2, false, false, false, true, true>(p, stream);
+  case Tile::k256:
+    return LaunchW<256, 256, 32, 3, 4, 2, true, false, false, true>(p, stream);
+  case Tile::k256Two:
+    return LaunchW<256, 256, 32, 2, 4, 2, true, false, false, true>(p, stream);
+  case Tile::k128x256:
+    return LaunchW<128, 256, 32, 3, 2, 4, true, false, false, true>(p, stream);
+  case Tile::kWide:
+    return LaunchW<128, 256, 32, 2, 2, 2, true, false, false, true>(p, stream);
+  case Tile::k128:
+    return LaunchW<128, 128, 64, 3, 2, 4, true, false, false, true>(p, stream);
+  case Tile::k64x128:
+    return LaunchW<64, 128, 64, 4, 2, 4, true, false, false, true>(p, stream);
+  case Tile::k64:
+    return LaunchW<64, 64, 64, 2, 2, 2, true, false, false, true>(p, stream);
+  case Tile::kNarrow:
+    return LaunchW<64, 64, 32, 2, 2, 2, true, false>(p, stream);
+  case Tile::kOne256:
+    return LaunchW<256, 256, 32, 4, 4, 2, false, false, false, true>(p, stream);
+  case Tile::kOneSlim:
+    return LaunchW<256, 128, 32, 3, 4, 2, false, false, false, true>(p, stream);
+  case Tile::kOne256x128:
+    return LaunchW<256, 128, 64, 3, 4, 2, false, false, false, true>(p, stream);
+  case Tile::kOne128:
+    return LaunchW<128, 128, 64, 4, 2, 4, false, false, false, true>(p, stream);
+  case Tile::kOne128Two:
+    return LaunchW<128, 128, 64, 2, 2, 4, false, false, false, true>(p, stream);
+  case Tile::kOne64x128:
+    return LaunchW<64, 128, 64, 3, 2, 2, false, false, false, true>(p, stream);
+  case Tile::kOne64:
+    return LaunchW<64, 64, 64, 3, 2, 2, false, false, false, true>(p, stream);
+  default:
+    return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace
 
-bool GemmLnFoldOk(const GemmParams &p) { return LnFoldTile(p) != LnTile::kNone; }
+bool GemmLnFoldOk(const GemmParams &p) {
+  // (The caller's parameters carry no LayerNorm yet: a consumer, or a
+  // residual GEMM as producer.)
+  if (p.out_mode != GEMM_OUT_BF16 && p.out_mode != GEMM_OUT_RESID_F32)
+    return false;
+  GemmParams q = p;
+  static const float one = 1.f;
+  if (q.out_mode == GEMM_OUT_RESID_F32)
+    q.out_gamma = &one;
+  else
+    q.fold_c = &one;
+  return LargeTile(q) != Tile::kNone;
+}
 
 // Split-K at few positions (64 x 64 tiles, K in 64-wide steps).  A GEMM
 // kernel here costs ~5 us however short its K loop, and a separate reduce
@@ -250,26 +447,23 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
     return fail("ldc too small");
   // Folded LayerNorm (see GemmParams): consumer and residual sides.
   const bool ln_res = p.out_mode == GEMM_OUT_RESID_F32 && (p.out_gamma || p.res_stats);
+  constexpr int kLnCols = kLnStatCols;
   if (p.fold_c && (!p.ln_stats || p.out_mode == GEMM_OUT_RESID_F32 || p.ln_width != p.K ||
-                   (p.ln_part != 64 && p.ln_part != 128) || p.K % (2 * p.ln_part) ||
-                   p.K > 128 * p.ln_part ||
-                   !Aligned(p.fold_c, 16) ||
+                   p.K % (2 * kLnCols) || p.K > 128 * kLnCols || !Aligned(p.fold_c, 16) ||
                    !Aligned(p.ln_stats, 16) || p.k_splits != 1))
-    return fail("folded LayerNorm consumer: ln_stats, fold_c (16-byte aligned), ln_part 64 or "
-                "128, K = ln_width a multiple of 2 ln_part up to 128 ln_part, one K slice, not "
-                "the residual mode");
+    return fail("folded LayerNorm consumer: ln_stats, fold_c (16-byte aligned), K = ln_width a "
+                "multiple of 256 up to 16384, one K slice, not the residual mode");
   if ((p.out_gamma || p.res_stats) && !ln_res)
     return fail("folded LayerNorm output / residual: residual mode only");
-  if (ln_res && (!p.resid16 || p.k_splits != 1 || p.ln_width != p.N ||
-                 (p.ln_part != 64 && p.ln_part != 128) || p.N % (2 * p.ln_part) ||
-                 p.N > 128 * p.ln_part ||
+  if (ln_res && (!p.resid16 || p.k_splits != 1 || p.ln_width != p.N || p.N % (2 * kLnCols) ||
+                 p.N > 128 * kLnCols ||
                  (p.res_stats && (!p.res_gamma || !p.res_beta || !Aligned(p.res_stats, 16) ||
                                   !Aligned(p.res_gamma, 16) || !Aligned(p.res_beta, 16))) ||
                  (p.out_gamma && (!p.out_stats || !Aligned(p.out_gamma, 16) ||
                                   !Aligned(p.out_stats, 8) || !p.C_lo))))
-    return fail("folded LayerNorm residual: split residual, one K slice, ln_part 64 or 128, "
-                "N = ln_width a multiple of 2 ln_part up to 128 ln_part, gamma / beta / stats "
-                "16-byte aligned, a bf16 lo output plane with out_gamma");
+    return fail("folded LayerNorm residual: split residual, one K slice, N = ln_width a "
+                "multiple of 256 up to 16384, gamma / beta / stats 16-byte aligned, a bf16 lo "
+                "output plane with out_gamma");
   if (p.C_lo8 && !(p.out_mode == GEMM_OUT_RESID_F32 && p.out_gamma) &&
       (p.out_mode != GEMM_OUT_BF16 || p.C_lo || p.split_n < p.N || p.k_splits != 1 ||
        p.ldc8 < p.N || p.ldc8 % 8 || !Aligned(p.C_lo8, 8)))
@@ -298,36 +492,26 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
            (p.out_mode != GEMM_OUT_RESID_F32 ||
             (p.resid16 ? Aligned(p.resid16, 16) && Aligned(p.resid16_lo, 16) && p.ldr % 8 == 0
                        : Aligned(p.resid, 16) && p.ldr % 4 == 0));
-  // fp8 lo correction: 256 x 256 tiles of eight waves, the hi pass on the
-  // four-stage single-bf16 pipelined ring (128 KiB), then the lo pass on two
-  // 64 KiB stages of code rows.
-  // A folded LayerNorm: only the instances that compile its epilogue.
-  if (p.fold_c || ln_res) {
-    switch (LnFoldTile(p)) {
-    case LnTile::kLo8:
-      return LaunchW<256, 256, 32, 4, 4, 2, false, false, false, true, true>(p, stream);
-    case LnTile::k256Beside:
-      return LaunchW<256, 256, 32, 2, 4, 2, true, false, false, true>(p, stream);
-    case LnTile::k256:
-      return LaunchW<256, 256, 32, 3, 4, 2, true, false, false, true>(p, stream);
-    case LnTile::k256x128:
-      return LaunchW<256, 128, 32, 2, 4, 2, true, false, false, true>(p, stream);
-    case LnTile::k64:
-      return LaunchW<64, 64, 32, 2, 2, 2, true, false>(p, stream);
-    case LnTile::k64x64:
-      return LaunchW<64, 64, 64, 2, 2, 2, true, false>(p, stream);
-    case LnTile::kSplitK:
-      if (!Aligned(p.partials, 16) || !p.vec || p.N % 4)
-        return fail("folded LayerNorm split over K: 16-byte aligned partials, vector stores");
-      break;  // the split-K launch below, its reduce applying the LayerNorm
-    default:
-      return fail("folded LayerNorm: split-precision activations, bf16 weights, one K slice, "
-                  "K % 64 == 0 and N a multiple of 256 (residual, BF16X2_FP8LO codes) or "
-                  "128 (or small-LDS tiles)");
-    }
+  // Split precision with bf16 weights, large shapes, and any folded
+  // LayerNorm: the tiles of LargeTile.  (BF16X2_FP8LO: 256 x 256 tiles of
+  // eight waves, the hi pass on the four-stage single-bf16 pipelined ring,
+  // 128 KiB, then the lo pass on two 64 KiB stages of code rows.)
+  const Tile tile = LargeTile(p);
+  if (tile == Tile::kSplitK) {
+    if (!Aligned(p.partials, 16) || !p.vec || p.N % 4)
+      return fail("folded LayerNorm split over K: 16-byte aligned partials, vector stores");
+  } else if (tile != Tile::kNone) {
+    const int rows = tile == Tile::kLo8 ? 0 : RowsFirst(p);
+    if (rows == 0)
+      return LaunchTile(tile, p, stream);
+    float us;
+    const hipError_t e = LaunchTile(p.A_lo ? Tile::k256 : Tile::kOne256, RowRange(p, 0, rows), stream);
+    const GemmParams rest = RowRange(p, rows, p.M - rows);
+    return e != hipSuccess ? e : LaunchTile(BestTile(rest, rest.M, &us), rest, stream);
+  } else if (p.fold_c || ln_res || lo8) {
+    return fail("folded LayerNorm or fp8 lo correction: split-precision activations, bf16 "
+                "weights, one K slice, K % 64 == 0 and N a multiple of the tile's width");
   }
-  if (lo8)
-    return LaunchW<256, 256, 32, 4, 4, 2, false, false, false, true, true>(p, stream);
   const bool split = p.A_lo != nullptr;
   const bool large = p.M >= kLargeRows && p.N >= 128;
   // Small problems (few positions): 64 x 64 tiles leave most CUs idle and
@@ -367,78 +551,25 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
   if (p.fold_c)
     return fail("folded LayerNorm: no tile for this shape");
   const int kslice = p.K / p.k_splits;
-  // Tile choice measured on MI355X at the BT4 body shapes (M = 16384): for
-  // K <= 1024, eight waves per workgroup on BK = 32 steps (split precision
-  // 128 x 128 tiles as 2 x 4 waves with two 48 KiB stages, bf16 256 x 128
-  // tiles as 4 x 2 waves with three 24 KiB stages); for longer K, four waves
-  // on BK = 64 (split 64 x 128, bf16 128 x 128).
-  // Whole rounds of 256 workgroups: 256 x 256 tiles of eight waves (4 x 2,
-  // 64 x 128 per wave) and a three-stage (split) or four-stage (bf16) LDS
-  // ring, 144 / 128 KiB, one workgroup per CU.  They halve the L2 traffic
-  // per MFMA of the 128-wide tiles; measured faster in the forward on the
-  // out-projection, FFN2 and smolgen-global shapes, slower on QKV (832 tiles,
-  // a partial last round) and FFN1 (384).  bf16 weights only (the fp8 path
-  // keeps two stages).
   const long big_tiles = static_cast<long>((p.M + 255) / 256) * ((p.N + 255) / 256);
   if (f8)
     return big_tiles % 256 == 0 ? LaunchW<256, 256, 64, 2, 4, 2, false, false, true>(p, stream)
                                 : LaunchW<128, 128, 64, 2, 2, 4, false, false, true>(p, stream);
-  if (GemmWholeRoundTiles(p)) {
-    // fp8 weights too: their e4m3 rows share the ring (40 / 24 KiB stages).
-    if (p.W8)
-      return split ? LaunchW<256, 256, 32, 3, 4, 2, true, true>(p, stream)
-                   : LaunchW<256, 256, 32, 4, 4, 2, false, true>(p, stream);
-    // Beside the smolgen chain (Q|K|V at large batches): two stages, so
-    // the chain's small-LDS tiles run on the same CUs instead of waiting for
-    // a round of these tiles to end (batch 256 forward 23.01k -> 23.55k
-    // positions/s with the chain on small-LDS tiles; two stages alone
-    // 23.15k, batch 1024 unchanged).
-    // bf16 weights: the software-pipelined main loop (PipelinedLoop).
-    // Isolated at batch 256, split precision: Q|K|V 223 -> 209 us, the
-    // out-projection 76.7 -> 70.7, FFN2 103.8 -> 93.6; single bf16 Q|K|V
-    // 112 -> 104; the batch-256 forward 23.15k -> 23.64k positions/s
-    // (bit-equal outputs: the MFMAs accumulate in the same order).
-    if (p.beside_chain && split)
-      return LaunchW<256, 256, 32, 2, 4, 2, true, false, false, true>(p, stream);
-    return split ? LaunchW<256, 256, 32, 3, 4, 2, true, false, false, true>(p, stream)
-                 : LaunchW<256, 256, 32, 4, 4, 2, false, false, false, true>(p, stream);
-  }
-  // Split precision with fewer 128 x 128 tiles than CUs (the out-projection
-  // and FFN at M = 2048 .. 3072): 64 x 64 tiles, four times the workgroups
-  // (out-projection at M = 2048: 13.5 instead of 25.4 us; batch 32 forward
-  // 3.02 -> 2.78 ms).  64 x 128 tiles between one and three rounds were
-  // faster in isolated launches but 2 % slower in the forward at batches 64
-  // and 96, so those keep 128 x 128.
-  const long tiles128 = static_cast<long>((p.M + 127) / 128) * ((p.N + 127) / 128);
-  if (large && kslice % 64 == 0) {
+  if (p.W8 && GemmWholeRoundTiles(p))
+    return split ? LaunchW<256, 256, 32, 3, 4, 2, true, true>(p, stream)
+                 : LaunchW<256, 256, 32, 4, 4, 2, false, true>(p, stream);
+  if (p.W8 && large && kslice % 64 == 0) {
+    const long tiles128 = static_cast<long>((p.M + 127) / 128) * ((p.N + 127) / 128);
     if (split && tiles128 < 256)
-      return Launch<64, 64, 64, 2, 2, 2, true>(p, stream);
-    if (kslice <= 1024 && split && !p.W8) {
-      // 256 x 128 tiles (eight 64 x 64 waves, two 40 KiB stages, two
-      // workgroups per CU) read 12 LDS fragments per 32 MFMAs, 128 x 128
-      // tiles 10 per 16; a 256 x 128 tile costs ~1.8 times a 128 x 128
-      // one, so it is taken when its rounds of 256 workgroups cost less and
-      // it fills at least one round.  Below one round (FFN1 at batches 48
-      // and 64, the out-projection at 96) it was 1-5 % slower, except for
-      // Q|K|V at 2048 rows (batch 32), where its 192 tiles leave CUs to the
-      // smolgen chain running beside it, the longer branch there.
-      // Measured forward: batch 32 2.72 -> 2.61 ms, 96 5.32 -> 5.26, 128
-      // 6.72 -> 6.66, 256 11.30 -> 11.16; 48 and 64 unchanged.
-      const long t256 = static_cast<long>((p.M + 255) / 256) * ((p.N + 127) / 128);
-      if ((t256 >= 256 || p.M <= 2048) &&
-          9 * ((t256 + 255) / 256) < 5 * ((tiles128 + 255) / 256))
-        return LaunchW<256, 128, 32, 2, 4, 2, true, false, false, true>(p, stream);
-    }
+      return LaunchW<64, 64, 64, 2, 2, 2, true, true>(p, stream);
     // Split precision with fp8 weights: BK = 64, whose stage holds the
     // e4m3 rows in LDS (at BK = 32 the 128 x 128 stage does not split
     // evenly over the waves).
     if (kslice <= 1024)
-      return split ? (p.W8 ? LaunchW<128, 128, 64, 2, 2, 4, true, true>(p, stream)
-                           : LaunchW<128, 128, 32, 2, 2, 4, true, false>(p, stream))
-             : p.W8 ? LaunchW<256, 128, 32, 2, 4, 2, false, true>(p, stream)
-                    : LaunchW<256, 128, 32, 3, 4, 2, false, false, false, true>(p, stream);
-    return split ? Launch<64, 128, 64, 2, 2, 2, true>(p, stream)
-                 : Launch<128, 128, 64, 2, 2, 2, false>(p, stream);
+      return split ? LaunchW<128, 128, 64, 2, 2, 4, true, true>(p, stream)
+                   : LaunchW<256, 128, 32, 2, 4, 2, false, true>(p, stream);
+    return split ? LaunchW<64, 128, 64, 2, 2, 2, true, true>(p, stream)
+                 : LaunchW<128, 128, 64, 2, 2, 2, false, true>(p, stream);
   }
   // 64 x 64 tiles over the whole K (Q|K|V at 4-31 positions, the
   // out-projection and FFN at 16-31, the smolgen dense2 and global

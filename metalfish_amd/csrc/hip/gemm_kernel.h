@@ -63,9 +63,9 @@ __device__ __forceinline__ int Swz(int row, int chunk) {
 // mu and r = 1 / sqrt(var + eps) of row `row` of a folded LayerNorm from
 // its partial sums (width / part (sum x, sum x^2) pairs, added in order),
 // with the reference formula var = E[x^2] - mu^2 clamped at 0.
-__device__ __forceinline__ void RowLnStats(const float *stats, int width, int part, float eps,
-                                           int row, float &mu, float &r) {
-  const int pairs2 = width / (2 * part);
+__device__ __forceinline__ void RowLnStats(const float *stats, int width, float eps, int row,
+                                           float &mu, float &r) {
+  const int pairs2 = width / (2 * kLnStatCols);
   const f32x4 *q = reinterpret_cast<const f32x4 *>(stats) + static_cast<size_t>(row) * pairs2;
   float s = 0.f, s2 = 0.f;
   // Eight quads at a time, loaded together.
@@ -106,7 +106,7 @@ __device__ __forceinline__ void LoadVec8(const float *v, int col, float (&o)[8])
 // costs registers the 256 x 128 tiles do not have.)
 __device__ __forceinline__ void FoldLn8(const GemmParams &p, int row, int col, float (&v)[8]) {
   float mu, rr;
-  RowLnStats(p.ln_stats, p.ln_width, p.ln_part, p.ln_eps, row, mu, rr);
+  RowLnStats(p.ln_stats, p.ln_width, p.ln_eps, row, mu, rr);
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const f32x4 c = *reinterpret_cast<const f32x4 *>(p.fold_c + col + 4 * h);
@@ -133,7 +133,7 @@ __device__ __forceinline__ void Epilogue4(const GemmParams &p, int row, int col,
   if (LN && p.fold_c) {
     // Consumer of a folded LayerNorm (never in the residual mode).
     float mu, rr;
-    RowLnStats(p.ln_stats, p.ln_width, p.ln_part, p.ln_eps, row, mu, rr);
+    RowLnStats(p.ln_stats, p.ln_width, p.ln_eps, row, mu, rr);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       acc[r] = rr * (acc[r] - mu * (col + r < p.N ? p.fold_c[col + r] : 0.f));
@@ -501,12 +501,14 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
     }
   }
   const int ldsw = __builtin_amdgcn_readfirstlane(wave * LPW * 512);  // elements
+  auto fill_one = [&](int s, int slot, int j) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc[j], MFH_LDS_PTR(lds + slot * STAGE + ldsw + j * 512),
+                                             16, goff[j], s * (BK * 2), 0, 0);
+  };
   auto fill = [&](int s, int slot) {
-    std::uint16_t *d = lds + slot * STAGE + ldsw;
 #pragma unroll
     for (int j = 0; j < LPW; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc[j], MFH_LDS_PTR(d + j * 512), 16, goff[j],
-                                               s * (BK * 2), 0, 0);
+      fill_one(s, slot, j);
   };
 
   const int a_off = Swz<BK>(wm * (BM / WM) + fr, fc);
@@ -549,29 +551,54 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
   // every wait on those reads becomes lgkmcnt(0).
   __builtin_amdgcn_s_waitcnt(kWaitLgkm);
 
-  // Stage k + 1 visible, slot of stage k refilled with stage k + ST.
-  // (The lgkmcnt(0) wait is unconditional: a wait chosen between two
-  // branches leaves the wait-count pass a path with no wait at all, and it
-  // then waits for every read issued after the barrier.)
-  auto sync_next = [&](int k, int fslot) {
+  // Stage k + 1 visible and the slot of stage k free, for every wave.  In the
+  // steady loop the loads of the ST - 2 stages after k + 1 stay in flight;
+  // where no more are issued (the last ST steps), every load is waited for.
+  auto sync_next = [&](auto tag) {
+    __builtin_amdgcn_s_waitcnt(decltype(tag)::value ? kWaitKeep : kWaitAll);
+    asm volatile("s_barrier" ::: "memory");
+  };
+  // The same after step 0, whose later stages may be fewer than ST.  (The
+  // lgkmcnt(0) wait is unconditional: a wait chosen between two branches
+  // leaves the wait-count pass a path with no wait at all, and it then waits
+  // for every read issued after the barrier.)
+  auto sync_first = [&]() {
     __builtin_amdgcn_s_waitcnt(kWaitKeep);
-    if (k + ST - 1 >= KT)
+    if (KT < ST)
       __builtin_amdgcn_s_waitcnt(kWaitAll);
     asm volatile("s_barrier" ::: "memory");
-    if (k + ST < KT)
-      fill(k + ST, fslot);
   };
 
   bf16x8 w[TN];
-  // The last step reads nothing more: it is peeled off so that the steady
-  // loop's reads are unconditional and the wait counts stay exact.
-  using More = std::integral_constant<bool, true>;
-  using Last = std::integral_constant<bool, false>;
+  // Compile-time switches of a step: whether a next stage is read, and
+  // whether a later one is loaded.
+  using Yes = std::integral_constant<bool, true>;
+  using No = std::integral_constant<bool, false>;
+  // The loads of a stage are issued between the step's MFMA groups, evenly
+  // over G of them from the first one on.  Issued together behind the
+  // barrier (every wave of the workgroup at once), they held each wave's
+  // next MFMAs until the address unit had taken them: a 32-wide step of a
+  // 256 x 256 split tile took 1.07 us on an otherwise idle chip, now 0.90
+  // (0.85 is the MFMAs alone); isolated at 16384 rows, split precision, the
+  // out-projection 70.5 -> 67.6 us, FFN2 96.1 -> 91.6, Q|K|V 171 -> 165.
+  // (Two-stage rings wait for these loads at the end of the step: within its
+  // first quarter.)
+  constexpr int kGroups = SPLIT ? 2 * TN : TN;
+  constexpr int G = ST > 2 ? kGroups : kGroups / 4 > 0 ? kGroups / 4 : 1;
+  auto fill_part = [&](auto tag, int g, int s, int slot) {
+    if constexpr (decltype(tag)::value) {
+#pragma unroll
+      for (int j = (g * LPW + G - 1) / G; j < ((g + 1) * LPW + G - 1) / G && j < LPW; ++j)
+        fill_one(s, slot, j);
+    }
+  };
   int cslot = 0;  // slot of stage k
+  auto next_slot = [](int s) { return s + 1 == ST ? 0 : s + 1; };
   if constexpr (SPLIT) {
     // The loop is rotated so that its header follows the step's barrier,
     // whose lgkmcnt(0) already drained the reads: an iteration is the lo
-    // half of step k (reading stage k + 1) and the hi half of step k + 1.
+    // half of step k (reading stage k + 1) and the hi half of step k + 1,
+    // loading stage k + ST into the slot of stage k.
     bf16x8 ahi[TM], alo[TM];
     read_a(ahi, lds, 0);
 #pragma unroll
@@ -579,14 +606,14 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
       read_w(w[j], lds, j);
     // hi half of a step whose stage is `cur`: the step's lo fragments are
     // read behind its first MFMA group.
-    auto hi_half = [&](const std::uint16_t *cur) {
-      mfma_group(w[0], ahi, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      read_a(alo, cur, 1);
-      __builtin_amdgcn_sched_barrier(0);
+    auto hi_half = [&](auto load, const std::uint16_t *cur, int s, int slot) {
 #pragma unroll
-      for (int j = 1; j < TN; ++j) {
+      for (int j = 0; j < TN; ++j) {
         mfma_group(w[j], ahi, j);
+        __builtin_amdgcn_sched_barrier(0);
+        if (j == 0)
+          read_a(alo, cur, 1);
+        fill_part(load, TN + j, s, slot);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -595,38 +622,46 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
     // step rolls in behind its last MFMA.  (No read precedes the first
     // group: the wait-count pass waits for every outstanding LDS read
     // where the loop begins, and nothing is in flight there yet.)
-    auto lo_half = [&](auto tag, const std::uint16_t *nxt) {
-      constexpr bool more = decltype(tag)::value;
+    auto lo_half = [&](auto more, auto load, const std::uint16_t *nxt, int s, int slot) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         mfma_group(w[j], alo, j);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (more) {
+        if constexpr (decltype(more)::value) {
           if (j == 0)
             read_a(ahi, nxt, 0);
           read_w(w[j], nxt, j);
         }
+        fill_part(load, j, s, slot);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    hi_half(lds);
+    hi_half(No(), lds, 0, 0);
     if (KT > 1)
-      sync_next(0, 0);
-    for (int k = 0; k + 2 < KT; ++k) {
-      const int nslot = cslot + 1 == ST ? 0 : cslot + 1;
+      sync_first();
+    int k = 0;
+    for (; k + ST < KT; ++k) {
+      const int nslot = next_slot(cslot);
       const std::uint16_t *nxt = lds + nslot * STAGE;
-      lo_half(More(), nxt);
-      hi_half(nxt);
-      sync_next(k + 1, nslot);
+      lo_half(Yes(), Yes(), nxt, k + ST, cslot);
+      hi_half(Yes(), nxt, k + ST, cslot);
+      sync_next(Yes());
+      cslot = nslot;
+    }
+    for (; k + 2 < KT; ++k) {
+      const int nslot = next_slot(cslot);
+      const std::uint16_t *nxt = lds + nslot * STAGE;
+      lo_half(Yes(), No(), nxt, 0, 0);
+      hi_half(No(), nxt, 0, 0);
+      sync_next(No());
       cslot = nslot;
     }
     if (KT > 1) {
-      const int nslot = cslot + 1 == ST ? 0 : cslot + 1;
-      const std::uint16_t *nxt = lds + nslot * STAGE;
-      lo_half(More(), nxt);
-      hi_half(nxt);
+      const std::uint16_t *nxt = lds + next_slot(cslot) * STAGE;
+      lo_half(Yes(), No(), nxt, 0, 0);
+      hi_half(No(), nxt, 0, 0);
     }
-    lo_half(Last(), lds);
+    lo_half(No(), No(), lds, 0, 0);
   } else {
     // Single bf16: the step's activation fragments feed every MFMA group,
     // so the next step's go into a second set; the loop is rotated like
@@ -637,25 +672,26 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
 #pragma unroll
     for (int j = 0; j < TN; ++j)
       read_w(w[j], lds, j);
-    auto rest = [&](auto tag, const std::uint16_t *nxt) {
-      constexpr bool more = decltype(tag)::value;
+    auto rest = [&](auto more, auto load, const std::uint16_t *nxt, int s, int slot) {
       // Nothing is in flight here (the barrier's wait drained the reads);
       // saying so keeps the wait-count pass from draining mid-step.
       __builtin_amdgcn_s_waitcnt(kWaitLgkm);
-      if constexpr (more) {
+      if constexpr (decltype(more)::value) {
         read_a(an, nxt, 0);
         read_w(w[0], nxt, 0);
       }
+      fill_part(load, 0, s, slot);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 1; j < TN; ++j) {
         mfma_group(w[j], a, j);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (more)
+        if constexpr (decltype(more)::value)
           read_w(w[j], nxt, j);
+        fill_part(load, j, s, slot);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if constexpr (more) {
+      if constexpr (decltype(more)::value) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
           a[i] = an[i];
@@ -666,19 +702,189 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
     mfma_group(w[0], a, 0);
     __builtin_amdgcn_sched_barrier(0);
     if (KT > 1)
-      sync_next(0, 0);
-    for (int k = 0; k + 2 < KT; ++k) {
-      const int nslot = cslot + 1 == ST ? 0 : cslot + 1;
-      rest(More(), lds + nslot * STAGE);
-      sync_next(k + 1, nslot);
+      sync_first();
+    int k = 0;
+    for (; k + ST < KT; ++k) {
+      const int nslot = next_slot(cslot);
+      rest(Yes(), Yes(), lds + nslot * STAGE, k + ST, cslot);
+      sync_next(Yes());
       cslot = nslot;
     }
-    if (KT > 1) {
-      const int nslot = cslot + 1 == ST ? 0 : cslot + 1;
-      rest(More(), lds + nslot * STAGE);
+    for (; k + 2 < KT; ++k) {
+      const int nslot = next_slot(cslot);
+      rest(Yes(), No(), lds + nslot * STAGE, 0, 0);
+      sync_next(No());
+      cslot = nslot;
     }
-    rest(Last(), lds);
+    if (KT > 1)
+      rest(Yes(), No(), lds + next_slot(cslot) * STAGE, 0, 0);
+    rest(No(), No(), lds, 0, 0);
   }
+}
+
+// Software-pipelined main loop over BK = 64 stages (bf16 weights), for tiles
+// too small to hide a barrier and an LDS latency behind one 32-wide K step's
+// MFMAs.  A stage is two 32-wide substeps and has one barrier; the fragments
+// are double-buffered in registers: a substep's MFMAs run on one set while
+// the other set is read for the next substep, a whole substep ahead of its
+// use.  A 32-wide step of a 128 x 128 split tile takes 0.28 us this way
+// (0.21 the MFMAs alone) against 0.39 in PipelinedLoop and 0.6 lock-step.
+// Isolated, split precision, best of the tiles before and now: 2048 rows
+// out-projection 15.1 -> 12.6 us, FFN2 20.0 -> 15.7, 4096 rows 22.8 -> 19.1
+// and 30.1 -> 24.6, Q|K|V 57.9 -> 45.9.  (More stages than the tables in
+// gemm.hip give change nothing: the loop is not bound by the loads'
+// latency.)
+//
+// The barrier stands between a stage's substeps: there the wave's reads of
+// the stage are complete (its second set was read during the first
+// substep), so past the barrier the stage's slot takes stage t + ST, and the
+// loads of stage t + 1, waited for in front of it, are visible to every
+// wave.  The loop is rotated to begin right after the barrier, where no LDS
+// read is in flight.  The loads of a stage are spread over the MFMA groups
+// of an iteration.
+template <int BM, int BN, int ST, int WM, int WN, bool SPLIT, int STAGE>
+__device__ __forceinline__ void DoubleBufferLoop(const GemmParams &p, std::uint16_t *lds, int m0,
+                                                 int n0, int k_begin, int KT,
+                                                 f32x4 (&acc)[BM / WM / 16][BN / WN / 16]) {
+  constexpr int BK = 64, NWAVES = WM * WN;
+  constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
+  constexpr int P = SPLIT ? 2 : 1;
+  constexpr int RPL = 8;  // rows of 128 bytes per 1 KiB wave-load
+  constexpr int LPW = STAGE * 2 / 1024 / NWAVES;
+  static_assert(BM % (RPL * NWAVES) == 0 && BN % (RPL * NWAVES) == 0,
+                "the wave-loads of one index stay inside one operand");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int fr = lane & 15, fc = lane >> 4;
+
+  // Wave-load j of wave w covers stage rows (j NWAVES + w) 8 .. + 7 (A rows,
+  // then A_lo, then W), lane l taking row l / 8 and the logical chunk that
+  // belongs in its slot.
+  const __amdgpu_buffer_rsrc_t ra = BufferRsrc(p.A);
+  const __amdgpu_buffer_rsrc_t ral = BufferRsrc(SPLIT ? p.A_lo : p.A);
+  const __amdgpu_buffer_rsrc_t rw = BufferRsrc(p.W);
+  unsigned goff[LPW];
+#pragma unroll
+  for (int j = 0; j < LPW; ++j) {
+    const int first = j * NWAVES * RPL;  // row of wave 0's load
+    const int row = first + wave * RPL + lane / 8;
+    const int chunk = Swz64Chunk(row, lane % 8);
+    if (first < P * BM)
+      goff[j] = 2u * (static_cast<unsigned>(min(m0 + row % BM, p.M - 1)) * p.lda + k_begin +
+                      chunk * 8);
+    else
+      goff[j] = 2u * (static_cast<unsigned>(min(n0 + row - P * BM, p.N - 1)) * p.ldw + k_begin +
+                      chunk * 8);
+  }
+  const int ldsw = __builtin_amdgcn_readfirstlane(wave * 512);  // elements
+  auto fill_one = [&](int s, int slot, int j) {
+    const int first = j * NWAVES * RPL;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        first < BM ? ra : first < P * BM ? ral : rw,
+        MFH_LDS_PTR(lds + slot * STAGE + ldsw + j * NWAVES * 512), 16, goff[j], s * (BK * 2), 0, 0);
+  };
+
+  // Fragment (plane q, row tile i) of substep kk, and weight fragment j.
+  // (Rows 16 apart share their swizzle.)
+  const int a_row = wm * (BM / WM) + fr, w_row = P * BM + wn * (BN / WN) + fr;
+  const int a_off[2] = {Swz<BK>(a_row, fc), Swz<BK>(a_row, 4 + fc)};
+  const int w_off[2] = {Swz<BK>(w_row, fc), Swz<BK>(w_row, 4 + fc)};
+  struct Set {
+    bf16x8 a[P][TM], w[TN];
+  };
+  constexpr int kReads = P * TM + TN;
+  // Read number r of a set: the weight fragment and hi rows that the first
+  // MFMAs take, then the rest.
+  auto read_one = [&](Set &f, const std::uint16_t *base, int kk, int r) {
+    if (r < TN)
+      f.w[r] = *reinterpret_cast<const bf16x8 *>(base + w_off[kk] + r * 16 * BK);
+    else
+      f.a[(r - TN) / TM][(r - TN) % TM] = *reinterpret_cast<const bf16x8 *>(
+          base + a_off[kk] + ((r - TN) / TM * BM + (r - TN) % TM * 16) * BK);
+  };
+  constexpr int kVmKeep = (ST - 2) * LPW;
+  constexpr int kPro = (ST - 1) * LPW;
+  static_assert(kPro < 64, "vmcnt holds at most 63");
+  constexpr int kWaitKeep = (kVmKeep & 15) | ((kVmKeep >> 4) << 14) | (7 << 4);
+  constexpr int kWaitAll = 7 << 4;
+  constexpr int kWaitPro = (kPro & 15) | ((kPro >> 4) << 14) | (7 << 4) | (15 << 8);
+  using Yes = std::integral_constant<bool, true>;
+  using No = std::integral_constant<bool, false>;
+  constexpr int G = P * TN;  // MFMA groups of a substep
+  // A substep on set `f`, reading set `n` from substep kk of `base` and
+  // issuing half `h` of the loads of stage s.
+  auto substep = [&](const Set &f, auto more, Set &n, const std::uint16_t *base, int kk, auto load,
+                     int h, int s, int slot) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int q = g / TN, j = g % TN;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[j], f.a[q][i], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (decltype(more)::value) {
+        // All reads within the first three quarters of the groups.
+        constexpr int GR = G * 3 / 4 > 0 ? G * 3 / 4 : 1;
+#pragma unroll
+        for (int r = (g * kReads + GR - 1) / GR; r < ((g + 1) * kReads + GR - 1) / GR && r < kReads;
+             ++r)
+          read_one(n, base, kk, r);
+      }
+      if constexpr (decltype(load)::value) {
+#pragma unroll
+        for (int l = ((h * G + g) * LPW + 2 * G - 1) / (2 * G);
+             l < ((h * G + g + 1) * LPW + 2 * G - 1) / (2 * G) && l < LPW; ++l)
+          fill_one(s, slot, l);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+#pragma unroll
+  for (int s = 0; s < ST; ++s)
+    if (s < KT) {
+#pragma unroll
+      for (int j = 0; j < LPW; ++j)
+        fill_one(s, s, j);
+    }
+  if (KT >= ST)
+    __builtin_amdgcn_s_waitcnt(kWaitPro);
+  else
+    __builtin_amdgcn_s_waitcnt(0);
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC00F | (7 << 4));  // lgkmcnt(0): no scalar load pending
+  Set f0, f1;
+#pragma unroll
+  for (int r = 0; r < kReads; ++r)
+    read_one(f0, lds, 0, r);
+  substep(f0, Yes(), f1, lds, 1, No(), 0, 0, 0);
+  // (Unconditional lgkmcnt(0), see PipelinedLoop.)
+  __builtin_amdgcn_s_waitcnt(kWaitKeep);
+  if (KT < ST)
+    __builtin_amdgcn_s_waitcnt(kWaitAll);
+  asm volatile("s_barrier" ::: "memory");
+  int t = 0, cslot = 0;
+  auto next_slot = [](int s) { return s + 1 == ST ? 0 : s + 1; };
+  for (; t + ST < KT; ++t) {
+    const int nslot = next_slot(cslot);
+    const std::uint16_t *nxt = lds + nslot * STAGE;
+    substep(f1, Yes(), f0, nxt, 0, Yes(), 0, t + ST, cslot);
+    substep(f0, Yes(), f1, nxt, 1, Yes(), 1, t + ST, cslot);
+    __builtin_amdgcn_s_waitcnt(kWaitKeep);
+    asm volatile("s_barrier" ::: "memory");
+    cslot = nslot;
+  }
+  for (; t + 1 < KT; ++t) {
+    const int nslot = next_slot(cslot);
+    const std::uint16_t *nxt = lds + nslot * STAGE;
+    substep(f1, Yes(), f0, nxt, 0, No(), 0, 0, 0);
+    substep(f0, Yes(), f1, nxt, 1, No(), 0, 0, 0);
+    __builtin_amdgcn_s_waitcnt(kWaitAll);
+    asm volatile("s_barrier" ::: "memory");
+    cslot = nslot;
+  }
+  substep(f1, No(), f0, lds, 0, No(), 0, 0, 0);
 }
 
 // The fp8 lo-correction pass of the BF16X2_FP8LO precision, run after the
@@ -783,9 +989,8 @@ __device__ __forceinline__ void Lo8Loop(const GemmParams &p, std::uint16_t *lds,
 
 template <int BM, int BN, int BK, int ST, int WM, int WN, bool SPLIT, int MODE, int ACT,
           bool W8, bool F8 = false, bool PIPE = false, bool LO8 = false, bool LN = false>
-// (The folded-LayerNorm 256 x 128 tiles are held to 128 VGPRs, two
-// workgroups per CU like the others of that shape.)
-__global__ __launch_bounds__(WM *WN * 64, (LN && BM == 256 && BN == 128) ? 4 : 1) void GemmKernel(
+// (Pipelined tiles of four waves: registers for two workgroups per CU.)
+__global__ __launch_bounds__(WM *WN * 64, PIPE && WM * WN == 4 ? 2 : 1) void GemmKernel(
     GemmParams p) {
   constexpr int NWAVES = WM * WN;
   constexpr int WTM = BM / WM, WTN = BN / WN;
@@ -807,7 +1012,7 @@ __global__ __launch_bounds__(WM *WN * 64, (LN && BM == 256 && BN == 128) ? 4 : 1
   // dimensions halved.
   static_assert(!F8 || (BK == 64 && !SPLIT && !W8), "fp8 activations: BK = 64 bytes pairs");
   static_assert(BK == 32 || BK == 64, "BK is 32 or 64");
-  static_assert(!PIPE || (!W8 && !F8 && BK == 32), "pipelined loop: bf16 weights, BK = 32");
+  static_assert(!PIPE || (!W8 && !F8), "pipelined loops: bf16 weights");
   static_assert(!LO8 || (PIPE && !SPLIT), "fp8 lo correction follows the single-plane hi pass");
   static_assert(LOADS % NWAVES == 0, "stage loads must split evenly over waves");
   constexpr int LPW = LOADS / NWAVES;
@@ -922,7 +1127,10 @@ __global__ __launch_bounds__(WM *WN * 64, (LN && BM == 256 && BN == 128) ? 4 : 1
 
   if constexpr (PIPE) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    PipelinedLoop<BM, BN, BK, ST, WM, WN, SPLIT, STAGE>(p, lds, m0, n0, k_begin, KT, acc);
+    if constexpr (BK == 64)
+      DoubleBufferLoop<BM, BN, ST, WM, WN, SPLIT, STAGE>(p, lds, m0, n0, k_begin, KT, acc);
+    else
+      PipelinedLoop<BM, BN, BK, ST, WM, WN, SPLIT, STAGE>(p, lds, m0, n0, k_begin, KT, acc);
     if constexpr (LO8)
       Lo8Loop<BM, BN, WM, WN, 2>(p, lds, m0, n0, acc);
 #endif
@@ -1124,11 +1332,9 @@ __global__ __launch_bounds__(WM *WN * 64, (LN && BM == 256 && BN == 128) ? 4 : 1
   constexpr int THREADS = NWAVES * 64;
   float ln_c0 = 0.f, ln_c1 = 0.f, ln_c2 = 0.f;
   bool ln_on = false;
-  // Load rounds issued before the staging: on 256-wide tiles all of them
-  // for rows of up to 4 quads (width 1024), wider rows load the rest in the
-  // staging; 128-wide tiles load all there (their registers are full: the
-  // FFN1 forward at batch 256 measured 0.9-1.9 % faster so).
-  constexpr int kLnPre = LN && BN == 256 ? (BM * 4 + THREADS - 1) / THREADS : 0;
+  // Load rounds issued before the staging: all of them for rows of up to 4
+  // quads (width 1024); wider rows load the rest in the staging.
+  constexpr int kLnPre = LN ? (BM * 4 + THREADS - 1) / THREADS : 0;
   f32x4 ln_v[kLnPre > 0 ? kLnPre : 1] = {};
   int ln_q = 0, ln_g = 1, ln_rounds = 0;
   const float *st = nullptr;
@@ -1169,7 +1375,7 @@ __global__ __launch_bounds__(WM *WN * 64, (LN && BM == 256 && BN == 128) ? 4 : 1
     // (sum, sum^2) pairs, a power of two, 64 at most), the first kLnPre
     // rounds of loads issued here so they are in flight during the staging.
     if (st) {
-      ln_q = p.ln_width / (2 * p.ln_part);
+      ln_q = p.ln_width / (2 * kLnStatCols);
       ln_g = 1;
       while (ln_g < ln_q)
         ln_g <<= 1;
@@ -1321,18 +1527,17 @@ __global__ __launch_bounds__(WM *WN * 64, (LN && BM == 256 && BN == 128) ? 4 : 1
     }
     return;
   }
-  if constexpr (LN && MODE == GEMM_OUT_RESID_F32 && (BN == 256 || BN == 64) &&
+  if constexpr (LN && MODE == GEMM_OUT_RESID_F32 && BN >= kLnStatCols &&
                 GemmLnEpilogueOk<BN, THREADS, RB>()) {
     if (PIPE || p.out_gamma || p.res_stats) {
       // Residual mode with a folded LayerNorm on either side (whole tiles,
       // checked by the launcher): the residual is LN(x) of x o gamma rows
       // (res_stats), and/or the result x = resid + alpha (acc + b) leaves
       // as x o out_gamma in bf16 hi + lo (+ e4m3 codes) with the partial
-      // sums of x over each block of kPart columns (128 on 256-wide tiles,
-      // 64 on 64-wide ones): a block is kPart / 8 consecutive lanes of one
-      // row (8 columns each), summed by shuffles in a fixed order.  A
-      // thread keeps one column group for the whole tile.
-      constexpr int kPartLanes = BN == 64 ? 8 : 16, kPart = 8 * kPartLanes;
+      // sums of x over each block of kPart columns: a block is kPart / 8
+      // consecutive lanes of one row (8 columns each), summed by shuffles in
+      // a fixed order.  A thread keeps one column group for the whole tile.
+      constexpr int kPart = kLnStatCols, kPartLanes = kPart / 8;
       int c8, r0;
       group_of(tid, r0, c8);
       const int col = n0 + c8;
@@ -1436,11 +1641,11 @@ hipError_t LaunchVariant(const GemmParams &p, hipStream_t stream) {
   auto kernel = GemmKernel<BM, BN, BK, ST, WM, WN, SPLIT, MODE, ACT, W8, F8, PIPE, LO8, LN>;
   constexpr int kRb = StagedRows<BM, BN, ST, GemmStageBytes<BM, BN, BK, WM, WN, SPLIT, W8>()>();
   if constexpr (MODE == GEMM_OUT_RESID_F32) {
-    // The folded-LayerNorm residual epilogue takes whole 256-wide tiles.
-    // (Partial sums per 128 columns on 256-wide tiles, per 64 on 64-wide.)
+    // The folded-LayerNorm residual epilogue takes whole 128- or 256-wide
+    // tiles.
     if ((p.out_gamma || p.res_stats) &&
-        !(LN && (BN == 256 || BN == 64) && GemmLnEpilogueOk<BN, WM * WN * 64, kRb>() &&
-          p.vec8 && p.N % BN == 0 && p.ln_part == (BN == 64 ? 64 : 128)))
+        !(LN && BN >= kLnStatCols && GemmLnEpilogueOk<BN, WM * WN * 64, kRb>() && p.vec8 &&
+          p.N % BN == 0))
       return hipErrorInvalidValue;
     if (LN && PIPE && !p.out_gamma && !p.res_stats)
       return hipErrorInvalidValue;
@@ -1482,9 +1687,10 @@ hipError_t LaunchW(const GemmParams &p, hipStream_t stream) {
   constexpr bool kLn = !W8 && !F8 && (SPLIT || LO8) && (PIPE || (BM == 64 && BN == 64));
   if (p.fold_c || p.out_gamma || p.res_stats) {
     if constexpr (kLn) {
-      if (p.k_splits == 1 && p.out_mode == GEMM_OUT_RESID_F32)
-        return LaunchVariant<BM, BN, BK, ST, WM, WN, SPLIT, GEMM_OUT_RESID_F32, ACT_NONE, W8, F8,
-                             PIPE, LO8, true>(p, stream);
+      if constexpr (BN >= kLnStatCols)
+        if (p.k_splits == 1 && p.out_mode == GEMM_OUT_RESID_F32)
+          return LaunchVariant<BM, BN, BK, ST, WM, WN, SPLIT, GEMM_OUT_RESID_F32, ACT_NONE, W8,
+                               F8, PIPE, LO8, true>(p, stream);
       if (p.k_splits == 1 && p.out_mode == GEMM_OUT_BF16 && p.act == ACT_NONE)
         return LaunchVariant<BM, BN, BK, ST, WM, WN, SPLIT, GEMM_OUT_BF16, ACT_NONE, W8, F8,
                              PIPE, LO8, true>(p, stream);

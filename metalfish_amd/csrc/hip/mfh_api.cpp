@@ -105,18 +105,22 @@ constexpr int kSmolgenSideRows = 1088;
 // BF16X2_FP8LO: the fp8 lo correction runs from this many token rows (128
 // positions); below, the forward is the BF16X2 one.
 constexpr int kLo8MinRows = 8192;
-// From this many token rows (256 positions) the body's residual LayerNorms
+// From this many token rows (24 positions) the body's residual LayerNorms
 // are folded into the GEMMs around them (GemmParams: the residual GEMMs write
 // x o gamma with per-row partial sums, Q|K|V, the compression and FFN1 take
-// the LayerNorm in their epilogue, the next residual rebuilds it), where
-// the residual GEMMs (N = E) take whole rounds of 256 x 256 tiles.
-constexpr long kFoldRows = 16384;
-// From this many token rows (24 positions), while the residual GEMMs take
-// 64 x 64 tiles over the whole K (up to 62 positions at E = 1024), the same
-// folds run on those tiles (partial sums per 64 columns): LN1 (out-projection -> FFN1 and FFN2) and LN2 (FFN2
-// -> Q|K|V on 256 x 128 tiles, the compression split over K with the
-// LayerNorm applied by its reduce, and the next out-projection).
-constexpr long kFoldLn1Rows = 1536;
+// the LayerNorm in their epilogue, the next residual rebuilds it).
+constexpr long kFoldRows = 1536;
+// (Fold measured against the LayerNorm kernels, one box: batch 48 3042 ->
+// 2777 us, 100 5287 -> 4999, 200 8699 -> 8234, 300 13181 -> 12463, 600 25877
+// -> 24432, 1000 41469 -> 39378.)  Very large residual streams whose N = E
+// GEMMs stop just short of whole rounds of 256 x 256 tiles keep the
+// kernels, as they always did (from kFoldShortElements elements and the
+// last round 9 / 10 full on).
+constexpr long kFoldShortElements = 32000000;
+bool StopsShortOfWholeRounds(long rows, long width) {
+  const long last = (rows + 255) / 256 * ((width + 255) / 256) % 256;
+  return rows * width >= kFoldShortElements && 10 * last >= 9 * 256;
+}
 
 std::uint16_t ToBf16(float f) {
   std::uint32_t u;
@@ -272,8 +276,8 @@ struct mfh_net {
   // offset of its e4m3 codes.
   std::map<size_t, size_t> lo8_codes;
   // The body's fold constants were packed (Layer::qkv_fold / ffn1_fold),
-  // for kFoldRows (has_fold) or kFoldLn1Rows (has_fold1) token rows.
-  bool has_fold = false, has_fold1 = false;
+  // for kFoldRows token rows.
+  bool has_fold = false;
   size_t head_b, qk_b, promo, val1_b, val2_w, val2_b, gather;
   size_t head_w[2], qk_w[2], val1_w[2];
   size_t mov_b = 0, mov1_b = 0, mov2_w = 0, mov2_b = 0;  // moves-left head
@@ -894,11 +898,11 @@ int Pack(mfh_net *net, Loader &ld, Blob &blob) {
       return rc;
   }
   // Folded residual LayerNorms of the body (split precisions, nets sized
-  // for kFoldLn1Rows token rows): Q|K|V (+ compression) of layer i > 0 over
+  // for kFoldRows token rows): Q|K|V (+ compression) of layer i > 0 over
   // layer i - 1's LN2, FFN1 of every layer over its LN1.
   const long net_rows = static_cast<long>(net->max_batch) * kSquares;
   if (d.fold_ln && d.split && !d.fp8_act && !d.fused_ln && d.E % (2 * mfh::kLnStatCols) == 0 &&
-      net_rows >= kFoldLn1Rows) {
+      net_rows >= kFoldRows) {
     const int qrows = 3 * E + (d.smolgen ? d.C : 0);
     for (int i = 0; i < d.L; ++i) {
       Layer &L = net->layers[i];
@@ -912,8 +916,7 @@ int Pack(mfh_net *net, Loader &ld, Blob &blob) {
       AddLnFold(blob, L.ffn1_w, net->fp8, flo8, d.F, E, L.ln1_g, L.ln1_b, L.ffn1_b,
                 L.ffn1_fold);
     }
-    net->has_fold = net_rows >= kFoldRows;
-    net->has_fold1 = true;
+    net->has_fold = true;
   }
   // Policy encoder layers (weights.cpp:188-203), no smolgen.
   net->pol_layers.resize(d.PL);
@@ -1067,7 +1070,7 @@ size_t PlanLayout(const Dims &d, int batch, size_t splitk_floats, bool side,
   // e4m3 lo parts of the encoder GEMM inputs (BF16X2_FP8LO), at the batches
   // whose forward uses them.
   if (d.fold_ln && d.split && !d.fp8_act && !d.fused_ln &&
-      d.E % (2 * mfh::kLnStatCols) == 0 && M >= static_cast<size_t>(kFoldLn1Rows)) {
+      d.E % (2 * mfh::kLnStatCols) == 0 && M >= static_cast<size_t>(kFoldRows)) {
     // Per-row partial sums of the folded LayerNorms' rows (LN2: "st_act",
     // LN1: "st_mid"), per 64 columns at most.
     add("st_act", M * (d.E / 64) * 2 * 4);
@@ -1314,21 +1317,12 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
   const bool lo8_act =
       lo8 && (whole_round(M, 3 * E) || whole_round(M, d.F) || (d.input_ffn && whole_round(M, d.Fi)));
   // The body's residual LayerNorms folded into the GEMMs around them (see
-  // kFoldRows): the whole forward (a single debug layer keeps them), where
-  // the residual GEMMs take whole rounds of 256 x 256 tiles.
+  // kFoldRows): the whole forward (a single debug layer keeps them).
   // (Checked below: every GEMM around them must have a tile that compiles
   // the folded epilogue.)
-  bool fold = net->has_fold && full && ws.Has("st_act") && whole_round(M, E) &&
-              M >= kSmolgenSideRows;
-  // Below whole rounds (kFoldLn1Rows on): LN1 on the 64 x 64 residual
-  // tiles (partial sums per 64 columns), and LN2 too where its consumers
-  // have tiles that fold it (fold2).
-  bool fold1 = !fold && net->has_fold1 && full && ws.Has("st_mid") && M >= kFoldLn1Rows;
-  bool fold2 = fold1 && ws.Has("st_act") && M >= kSmolgenSideRows;
+  bool fold = net->has_fold && full && ws.Has("st_act") && M >= kFoldRows &&
+              !StopsShortOfWholeRounds(M, E);
   float *st_act = nullptr, *st_mid = nullptr;
-  // Columns per partial sum: 128 on the whole-round 256-wide tiles, 64 on
-  // the 64-wide ones (set with the fold below).
-  int ln_part = 128;
   auto ln = [&](const float *x, int rows, int width, float eps, const float *g, const float *b,
                 float *y32, const std::string &y16) {
     mfh::LayerNormParams lp;
@@ -1475,7 +1469,6 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
     p.ldr = E;
     p.alpha = alpha;
     p.ln_width = E;
-    p.ln_part = ln_part;
     if (res_st) {
       p.res_stats = res_st;
       p.res_gamma = rg;
@@ -1719,10 +1712,10 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
     mfh::GemmParams pq = gemm("act", E, L.qkv_w, E, M, 3 * E, E, nullptr, mfh::ACT_NONE, bf16,
                               nullptr, nullptr, 3 * E);
     use_lo8(pq, "act", L.qkv_w);
-    pq.beside_chain = L.smolgen && ws.Has("splitk_sg") && mfh::GemmWholeRoundTiles(pq);
+    pq.beside_chain = L.smolgen && ws.Has("splitk_sg");
     mfh::GemmParams pc = gemm("act", E, L.qkv_w, E, M, d.C, E, nullptr, mfh::ACT_NONE, bf16,
                               nullptr, nullptr, d.C);
-    pc.small_lds = pq.beside_chain;
+    pc.small_lds = pq.beside_chain && mfh::GemmFillsCus(pq);
     mfh::GemmParams pf = gemm("act", E, L.ffn1_w, E, M, d.F, E, nullptr, d.act_ffn, bf16,
                               nullptr, nullptr, d.F);
     use_lo8(pf, "act", L.ffn1_w);
@@ -1735,43 +1728,10 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
     fold = (li == 0 || mfh::GemmLnFoldOk(pq)) && (li == 0 || !L.smolgen || mfh::GemmLnFoldOk(pc)) &&
            mfh::GemmLnFoldOk(pf) && mfh::GemmLnFoldOk(po) && mfh::GemmLnFoldOk(p2);
   }
-  // LN1: the out-projection (writing x o gamma1 with its sums), FFN1 (its
-  // consumer) and FFN2 (rebuilding the residual) on 64-wide tiles.  LN2:
-  // FFN2 writing x o gamma2, Q|K|V and the compression (beside Q|K|V on
-  // the side stream) of the next layer as its consumers.
-  for (int li = 0; fold1 && li < d.L; ++li) {
-    const Layer &L = net->layers[li];
-    const int bf16 = mfh::GEMM_OUT_BF16, res = mfh::GEMM_OUT_RESID_F32;
-    mfh::GemmParams pf = gemm("act", E, L.ffn1_w, E, M, d.F, E, nullptr, d.act_ffn, bf16,
-                              nullptr, nullptr, d.F);
-    mfh::GemmParams po = gemm("ctx", E, L.out_w, E, M, E, E, nullptr, mfh::ACT_NONE, res,
-                              nullptr, nullptr, E);
-    mfh::GemmParams p2 = gemm("hid", d.F, L.ffn2_w, d.F, M, E, d.F, nullptr, mfh::ACT_NONE, res,
-                              nullptr, nullptr, E);
-    const mfh::GemmParams *ps[3] = {&pf, &po, &p2};
-    for (const mfh::GemmParams *q : ps)
-      fold1 = fold1 && !q->A_lo8 && mfh::GemmLnFoldOk(*q);
-    // (The residual tiles must be the 64-wide ones their sums assume.  FFN1
-    // takes 64 x 64 tiles with the fold, also above 42 positions at the BT4
-    // widths, where it takes 128 x 128 ones without it.)
-    auto t128 = [&](int n) { return static_cast<long>((M + 127) / 128) * ((n + 127) / 128); };
-    fold1 = fold1 && t128(E) < 256;
-    if (li > 0 && fold2) {
-      mfh::GemmParams pq = gemm("act", E, L.qkv_w, E, M, 3 * E, E, nullptr, mfh::ACT_NONE, bf16,
-                                nullptr, nullptr, 3 * E);
-      mfh::GemmParams pc = gemm("act", E, L.qkv_w, E, M, d.C, E, nullptr, mfh::ACT_NONE, bf16,
-                                nullptr, nullptr, d.C);
-      fold2 = !pq.A_lo8 && mfh::GemmLnFoldOk(pq) && (!L.smolgen || mfh::GemmLnFoldOk(pc));
-    }
-  }
-  fold2 = fold2 && fold1;
-  if (fold || fold2) {
+  if (fold) {
     st_act = ws.S<float>("st_act");
     st_mid = ws.S<float>("st_mid");
-  } else if (fold1) {
-    st_mid = ws.S<float>("st_mid");
   }
-  ln_part = fold ? 128 : 64;
   auto encoder_layer = [&](const Layer &L, int heads, int ffn, float eps_attn, float eps_ffn,
                            float alpha, bool body_out) -> int {
     // The smolgen chain (compression, dense1, LayerNorm, dense2, LayerNorm,
@@ -1790,9 +1750,9 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
     // previous layer's folded LN2 from layer 1 on; LN2 is folded except
     // after the last layer, whose LayerNorm the heads read.
     const bool body = li < d.L;
-    const bool fold_mid = (fold || fold1) && body;
-    const bool fold_in = (fold || fold2) && body && li > 0;
-    const bool fold_out = (fold || fold2) && body && !body_out;
+    const bool fold_mid = fold && body;
+    const bool fold_in = fold && body && li > 0;
+    const bool fold_out = fold && body && !body_out;
     const Layer *prev = fold_in ? &net->layers[li - 1] : nullptr;
     // A GEMM reading LN(x) of folded rows (x o gamma with stats st): the
     // LayerNorm in its epilogue with the fold constants {fold_c, bias'}.
@@ -1800,8 +1760,7 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
                              const size_t (&fc)[2], size_t skip) {
       p.ln_stats = st;
       p.ln_width = E;
-      p.ln_part = ln_part;
-      p.ln_eps = eps;
+        p.ln_eps = eps;
       p.fold_c = net->W<float>(fc[0]) + skip;
       p.bias = net->W<float>(fc[1]) + skip;
     };
@@ -1825,16 +1784,15 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
       pq.C2_lo = ws.Lo("comp");
       pq.ldc2 = d.C;
     }
-    // Beside the chain, Q|K|V on whole-round 256 x 256 tiles takes two LDS
-    // stages and the chain's GEMMs 24 KiB tiles, which then fit on the CUs
-    // that hold Q|K|V workgroups.  Where Q|K|V takes 256 x 128 tiles (80
-    // KiB), the chain's usual tiles already fit beside them and are faster
-    // (24 KiB tiles there: batch 24 -1.6 %, 32 -1.1 %, 96 -1.4 %).
-    const bool share_cus = L.smolgen && chain_beside && mfh::GemmWholeRoundTiles(pq);
+    // Beside the chain, Q|K|V takes tiles that leave LDS to it; where they
+    // hold every CU (GemmFillsCus), the chain's GEMMs take 24 KiB tiles,
+    // which fit beside them, elsewhere the usual ones are faster (24 KiB
+    // tiles at batch 32 +8 %, 64 +7 %, 100 -0.8 %, 200 -1.0 %, 300 -0.9 %).
+    const bool share_cus = L.smolgen && chain_beside && mfh::GemmFillsCus(pq);
     // BF16X2_FP8LO: the lo parts of Q|K|V as e4m3 codes (no fused smolgen
     // bias in that precision; Q|K|V without the compression columns).
     const bool qkv_codes = lo8 && !d.fused_bias && pq.N == 3 * E;
-    pq.beside_chain = share_cus;
+    pq.beside_chain = L.smolgen && chain_beside;
     mfh::AttentionParams ap;
     ap.qkv = ws.S<std::uint16_t>("qkv");
     ap.qkv_lo = ws.Lo("qkv");

@@ -1,0 +1,75 @@
+"""The GEMM tiles of the large shapes (from 1536 rows): every tile gives the
+bits of the 64 x 64 tiles that small shapes take, and forwards at batches
+where the choice of tile, a row split or the LayerNorm fold changes agree
+with small batches."""
+
+import dataclasses
+
+import numpy as np
+import pytest
+
+from metalfish_amd import backend, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(rng, shape, scale=1.0):
+    x = (rng.standard_normal(shape) * scale).astype(np.float32)
+    u = x.view(np.uint32)
+    return ((u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+
+
+# Rows and widths around the edges of 64-, 128- and 256-wide tiles, K of one
+# 64-wide stage, fewer and more stages than any ring holds.
+@pytest.mark.parametrize("m,n,k", [(1536, 128, 64), (1537, 130, 128), (1600, 1024, 320),
+                                   (2047, 1024, 1024), (4096, 1024, 1024), (4100, 1536, 1024),
+                                   (6400, 1024, 1536), (12800, 256, 192), (16385, 256, 64),
+                                   (16640, 1024, 256), (1536, 1056, 96)])
+@pytest.mark.parametrize("act", ["none", "mish"])
+def test_large_tiles_equal_small_ones(m, n, k, act):
+    """The MFMAs of an output accumulate over K in one order on every tile,
+    so a row's bits do not depend on how many rows the call has (the small
+    call's 64 x 64 tiles run over the whole K); float64 bounds the product:
+    at most K * 2^-24 of the summed magnitudes, with a factor 2 for the
+    products' own rounding, and mish's slope is below 1.1."""
+    rng = np.random.default_rng(m * 7 + n + k)
+    a, w = _bits(rng, (m, k)), _bits(rng, (n, k), 1 / np.sqrt(k))
+    bias = rng.standard_normal(n).astype(np.float32)
+    out = backend.gemm_bf16(a, w, bias, act)
+    for lo in {0, m // 2, m - 70}:
+        rows = slice(lo, lo + 70)
+        small = backend.gemm_bf16(a[rows], w, bias, act)
+        assert np.array_equal(out[rows].view(np.uint32), small.view(np.uint32)), (lo, act)
+        x = (a[rows].astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+        y = (w.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+        z = x @ y.T + bias
+        bound = 1.1 * k * 2.0 ** -23 * (np.abs(x) @ np.abs(y).T + np.abs(bias)) + 1e-6
+        if act == "mish":
+            z = z * np.tanh(np.logaddexp(0.0, z))
+            bound = bound + 1e-5 * np.abs(z)
+        assert (np.abs(small - z) <= bound).all()
+
+
+@pytest.mark.parametrize("precision", ["bf16x2", "bf16x2_gemm", "bf16"])
+def test_batches_across_tile_rules_agree(precision):
+    """Two BT4-width layers: batches at the first folded one (24), odd ones,
+    one past a tile's whole rounds (65, 129, 257: the rows split over two
+    launches) and others agree with batch 4 position by position.  In bf16x2
+    to summation-order noise, 1e-4, as between any two batch sizes; the
+    other precisions round activations to bf16 (2^-9), so a last-bit
+    difference in a sum can move a logit by what the precision itself is off
+    by: 5e-3 and 3e-2 (their errors against the oracle)."""
+    tol = {"bf16x2": 1e-4, "bf16x2_gemm": 5e-3, "bf16": 3e-2}[precision]
+    spec = dataclasses.replace(synth.SPECS["bt4"], name="two", layers=2)
+    weights = synth.make_weights(spec, seed=2)
+    planes, _ = synth.playout_positions(4, seed=9)
+    net = backend.create_network(spec, weights, max_batch=321, device=0, precision=precision)
+    small = net.evaluate_batch(planes)
+    for batch in (24, 25, 33, 43, 64, 65, 100, 129, 200, 257, 300, 321):
+        idx = np.arange(batch) % 4
+        out = net.evaluate_batch(planes[idx])
+        err = np.abs(out["policy"] - small["policy"][idx]).max()
+        werr = np.abs(out["wdl"] - small["wdl"][idx]).max()
+        print(f"{precision} batch {batch}: policy {err:.2e} wdl {werr:.2e}", flush=True)
+        assert err <= tol and werr <= tol
+    net.close()
