@@ -70,15 +70,17 @@ hipError_t Reduce(const GemmParams &p, const float *part, int splits, hipStream_
   return LaunchReduce<GEMM_OUT_BF16, ACT_RUNTIME>(p, part, splits, stream);
 }
 
+// A tile with bf16 or fp8 weights on the pipelined loops.
 template <int BM, int BN, int BK, int ST, int WM, int WN, bool SPLIT>
-hipError_t Launch(const GemmParams &p, hipStream_t stream) {
-  // fp8 weights: the ring's stages when their rows go through LDS, else two
-  // (fragments from global memory).  bf16 weights over BK = 64: the
-  // double-buffered loop.
-  if (p.W8)
-    return LaunchW<BM, BN, BK, W8InLds<BM, BN, BK, WM, WN, SPLIT>() ? ST : 2, WM, WN, SPLIT,
-                   true>(p, stream);
-  return LaunchW<BM, BN, BK, ST, WM, WN, SPLIT, false, false, BK == 64>(p, stream);
+hipError_t LaunchPipe(const GemmParams &p, hipStream_t stream) {
+  return p.W8 ? LaunchW<BM, BN, BK, ST, WM, WN, SPLIT, true, false, true>(p, stream)
+              : LaunchW<BM, BN, BK, ST, WM, WN, SPLIT, false, false, true>(p, stream);
+}
+
+// 64 x 64 over BK = 32, lock-step (K a multiple of 32, or little LDS).
+template <bool SPLIT> hipError_t LaunchStep32(const GemmParams &p, hipStream_t stream) {
+  return p.W8 ? LaunchW<64, 64, 32, 2, 2, 2, SPLIT, true>(p, stream)
+              : LaunchW<64, 64, 32, 2, 2, 2, SPLIT, false>(p, stream);
 }
 
 bool Aligned(const void *ptr, std::uintptr_t bytes) {
@@ -101,13 +103,13 @@ bool GemmWholeRoundTiles(const GemmParams &p) {
 // (Split precision: two 128 x 256 tiles per CU.)
 bool GemmFillsCus(const GemmParams &p) {
   const long wide = static_cast<long>((p.M + 127) / 128) * ((p.N + 255) / 256);
-  return GemmWholeRoundTiles(p) || (p.A_lo && !p.W8 && p.M >= kLargeRows && wide >= 512);
+  return GemmWholeRoundTiles(p) || (p.A_lo && p.M >= kLargeRows && wide >= 512);
 }
 
 namespace {
 
-// The tiles of the GEMMs with bf16 weights from kLargeRows rows on.  Those of
-// split precision compile a folded LayerNorm's epilogue.
+// The tiles of the GEMMs from kLargeRows rows on (LDS sizes with bf16
+// weights).  Those of split precision compile a folded LayerNorm's epilogue.
 enum class Tile {
   kNone,
   kLo8,      // 256 x 256, BF16X2_FP8LO
@@ -185,6 +187,8 @@ Tile BestTile(const GemmParams &p, int M, float *us) {
   const auto consider = [&](const TileTime &t) {
     if (((p.fold_c || ln_res) && p.N % t.bn) || (ln_res && t.bn < kLnStatCols))
       return;
+    if (p.W8 && t.tile == Tile::kOneSlim)  // (its e4m3 stage is no whole wave-loads)
+      return;
     const float c = LaunchTime(t, M, p);
     if (best == Tile::kNone || c < *us) {
       best = t.tile;
@@ -221,12 +225,12 @@ int RowsFirst(const GemmParams &p) {
   return LaunchTime(whole, rows, p) + rest < 0.97f * one ? rows : 0;
 }
 
-// The tile of a large GEMM with bf16 weights, or of one with a folded
-// LayerNorm (kNone: none of these).
+// The tile of a large GEMM, or of one with a folded LayerNorm (kNone: none
+// of these).
 Tile LargeTile(const GemmParams &p) {
   const bool res = p.out_mode == GEMM_OUT_RESID_F32;
   const bool ln = p.fold_c || p.out_gamma || p.res_stats;
-  if (p.W8 || p.A8 || p.k_splits != 1 || p.K % 64)
+  if (p.A8 || p.k_splits != 1 || p.K % 64)
     return Tile::kNone;
   if (p.A_lo8)
     return !ln || p.N % 256 == 0 ? Tile::kLo8 : Tile::kNone;
@@ -234,7 +238,7 @@ Tile LargeTile(const GemmParams &p) {
     if (ln || p.M < kLargeRows || p.N < 128)
       return Tile::kNone;
     if (p.beside_chain)
-      return GemmWholeRoundTiles(p) ? Tile::kOne256 : Tile::kOneSlim;
+      return GemmWholeRoundTiles(p) ? Tile::kOne256 : p.W8 ? Tile::kOne128Two : Tile::kOneSlim;
     float us;
     return BestTile(p, p.M, &us);
   }
@@ -294,35 +298,35 @@ hipError_t LaunchTile(Tile t, const GemmParams &p, hipStream_t stream) {
   case Tile::kLo8:
     return LaunchW<256, 256, 32, 4, 4, 2, false, false, false, true, true>(p, stream);
   case Tile::k256:
-    return LaunchW<256, 256, 32, 3, 4, 2, true, false, false, true>(p, stream);
+    return LaunchPipe<256, 256, 32, 3, 4, 2, true>(p, stream);
   case Tile::k256Two:
-    return LaunchW<256, 256, 32, 2, 4, 2, true, false, false, true>(p, stream);
+    return LaunchPipe<256, 256, 32, 2, 4, 2, true>(p, stream);
   case Tile::k128x256:
-    return LaunchW<128, 256, 32, 3, 2, 4, true, false, false, true>(p, stream);
+    return LaunchPipe<128, 256, 32, 3, 2, 4, true>(p, stream);
   case Tile::kWide:
-    return LaunchW<128, 256, 32, 2, 2, 2, true, false, false, true>(p, stream);
+    return LaunchPipe<128, 256, 32, 2, 2, 2, true>(p, stream);
   case Tile::k128:
-    return LaunchW<128, 128, 64, 3, 2, 4, true, false, false, true>(p, stream);
+    return LaunchPipe<128, 128, 64, 3, 2, 4, true>(p, stream);
   case Tile::k64x128:
-    return LaunchW<64, 128, 64, 4, 2, 4, true, false, false, true>(p, stream);
+    return LaunchPipe<64, 128, 64, 4, 2, 4, true>(p, stream);
   case Tile::k64:
-    return LaunchW<64, 64, 64, 2, 2, 2, true, false, false, true>(p, stream);
+    return LaunchPipe<64, 64, 64, 2, 2, 2, true>(p, stream);
   case Tile::kNarrow:
-    return LaunchW<64, 64, 32, 2, 2, 2, true, false>(p, stream);
+    return LaunchStep32<true>(p, stream);
   case Tile::kOne256:
-    return LaunchW<256, 256, 32, 4, 4, 2, false, false, false, true>(p, stream);
+    return LaunchPipe<256, 256, 32, 4, 4, 2, false>(p, stream);
   case Tile::kOneSlim:
     return LaunchW<256, 128, 32, 3, 4, 2, false, false, false, true>(p, stream);
   case Tile::kOne256x128:
-    return LaunchW<256, 128, 64, 3, 4, 2, false, false, false, true>(p, stream);
+    return LaunchPipe<256, 128, 64, 3, 4, 2, false>(p, stream);
   case Tile::kOne128:
-    return LaunchW<128, 128, 64, 4, 2, 4, false, false, false, true>(p, stream);
+    return LaunchPipe<128, 128, 64, 4, 2, 4, false>(p, stream);
   case Tile::kOne128Two:
-    return LaunchW<128, 128, 64, 2, 2, 4, false, false, false, true>(p, stream);
+    return LaunchPipe<128, 128, 64, 2, 2, 4, false>(p, stream);
   case Tile::kOne64x128:
-    return LaunchW<64, 128, 64, 3, 2, 2, false, false, false, true>(p, stream);
+    return LaunchPipe<64, 128, 64, 3, 2, 2, false>(p, stream);
   case Tile::kOne64:
-    return LaunchW<64, 64, 64, 3, 2, 2, false, false, false, true>(p, stream);
+    return LaunchPipe<64, 64, 64, 3, 2, 2, false>(p, stream);
   default:
     return hipErrorInvalidValue;
   }
@@ -492,8 +496,7 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
            (p.out_mode != GEMM_OUT_RESID_F32 ||
             (p.resid16 ? Aligned(p.resid16, 16) && Aligned(p.resid16_lo, 16) && p.ldr % 8 == 0
                        : Aligned(p.resid, 16) && p.ldr % 4 == 0));
-  // Split precision with bf16 weights, large shapes, and any folded
-  // LayerNorm: the tiles of LargeTile.  (BF16X2_FP8LO: 256 x 256 tiles of
+  // Large shapes and any folded LayerNorm: the tiles of LargeTile.  (BF16X2_FP8LO: 256 x 256 tiles of
   // eight waves, the hi pass on the four-stage single-bf16 pipelined ring,
   // 128 KiB, then the lo pass on two 64 KiB stages of code rows.)
   const Tile tile = LargeTile(p);
@@ -509,8 +512,8 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
     const GemmParams rest = RowRange(p, rows, p.M - rows);
     return e != hipSuccess ? e : LaunchTile(BestTile(rest, rest.M, &us), rest, stream);
   } else if (p.fold_c || ln_res || lo8) {
-    return fail("folded LayerNorm or fp8 lo correction: split-precision activations, bf16 "
-                "weights, one K slice, K % 64 == 0 and N a multiple of the tile's width");
+    return fail("folded LayerNorm or fp8 lo correction: split-precision activations, one K "
+                "slice, K % 64 == 0 and N a multiple of the tile's width");
   }
   const bool split = p.A_lo != nullptr;
   const bool large = p.M >= kLargeRows && p.N >= 128;
@@ -536,10 +539,10 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
       q.k_splits = splits;
       q.vec = true;
       const bool small = p.small_lds && !p.W8;
-      const hipError_t e = small ? (split ? Launch<64, 64, 32, 2, 2, 2, true>(q, stream)
-                                          : Launch<64, 64, 32, 2, 2, 2, false>(q, stream))
-                           : split ? Launch<64, 64, 64, 3, 2, 2, true>(q, stream)
-                                   : Launch<64, 64, 64, 3, 2, 2, false>(q, stream);
+      const hipError_t e = small ? (split ? LaunchStep32<true>(q, stream)
+                                          : LaunchStep32<false>(q, stream))
+                           : split ? LaunchPipe<64, 64, 64, 3, 2, 2, true>(q, stream)
+                                   : LaunchPipe<64, 64, 64, 3, 2, 2, false>(q, stream);
       if (e != hipSuccess)
         return e;
       // The partials already carry the fp8 row scale.
@@ -555,22 +558,6 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
   if (f8)
     return big_tiles % 256 == 0 ? LaunchW<256, 256, 64, 2, 4, 2, false, false, true>(p, stream)
                                 : LaunchW<128, 128, 64, 2, 2, 4, false, false, true>(p, stream);
-  if (p.W8 && GemmWholeRoundTiles(p))
-    return split ? LaunchW<256, 256, 32, 3, 4, 2, true, true>(p, stream)
-                 : LaunchW<256, 256, 32, 4, 4, 2, false, true>(p, stream);
-  if (p.W8 && large && kslice % 64 == 0) {
-    const long tiles128 = static_cast<long>((p.M + 127) / 128) * ((p.N + 127) / 128);
-    if (split && tiles128 < 256)
-      return LaunchW<64, 64, 64, 2, 2, 2, true, true>(p, stream);
-    // Split precision with fp8 weights: BK = 64, whose stage holds the
-    // e4m3 rows in LDS (at BK = 32 the 128 x 128 stage does not split
-    // evenly over the waves).
-    if (kslice <= 1024)
-      return split ? LaunchW<128, 128, 64, 2, 2, 4, true, true>(p, stream)
-                   : LaunchW<256, 128, 32, 2, 4, 2, false, true>(p, stream);
-    return split ? LaunchW<64, 128, 64, 2, 2, 2, true, true>(p, stream)
-                 : LaunchW<128, 128, 64, 2, 2, 2, false, true>(p, stream);
-  }
   // 64 x 64 tiles over the whole K (Q|K|V at 4-31 positions, the
   // out-projection and FFN at 16-31, the smolgen dense2 and global
   // projection at some batches): from 256 rows up, or over K >= 1024, a
@@ -581,17 +568,15 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
   // beside the Q|K|V GEMM on the other stream) it was 1.7 % slower, and four
   // stages (one workgroup per CU) were slower at every batch.
   if (p.small_lds && !p.W8)
-    return split ? Launch<64, 64, 32, 2, 2, 2, true>(p, stream)
-                 : Launch<64, 64, 32, 2, 2, 2, false>(p, stream);
+    return split ? LaunchStep32<true>(p, stream) : LaunchStep32<false>(p, stream);
   if (kslice % 64 == 0) {
     if (p.M >= 256 || kslice >= 1024)
-      return split ? Launch<64, 64, 64, 3, 2, 2, true>(p, stream)
-                   : Launch<64, 64, 64, 3, 2, 2, false>(p, stream);
-    return split ? Launch<64, 64, 64, 2, 2, 2, true>(p, stream)
-                 : Launch<64, 64, 64, 2, 2, 2, false>(p, stream);
+      return split ? LaunchPipe<64, 64, 64, 3, 2, 2, true>(p, stream)
+                   : LaunchPipe<64, 64, 64, 3, 2, 2, false>(p, stream);
+    return split ? LaunchPipe<64, 64, 64, 2, 2, 2, true>(p, stream)
+                 : LaunchPipe<64, 64, 64, 2, 2, 2, false>(p, stream);
   }
-  return split ? Launch<64, 64, 32, 2, 2, 2, true>(p, stream)
-               : Launch<64, 64, 32, 2, 2, 2, false>(p, stream);
+  return split ? LaunchStep32<true>(p, stream) : LaunchStep32<false>(p, stream);
 }
 
 }  // namespace mfh

@@ -20,11 +20,11 @@
 // ends up holding four consecutive output columns of one row: the epilogue
 // stores 8 bytes (bf16) or 16 bytes (fp32) per lane instead of 2 or 4.
 //
-// FP8 weights (W8): the weight tile skips LDS.  Each wave loads its own
-// fragments (8 e4m3 codes = 8 bytes per lane) from global memory one K step
-// ahead, converts them exactly to bf16 with v_cvt_scalef32_pk_bf16_fp8, and
-// the row scale multiplies the accumulators in the epilogue (or the split-K
-// partials).
+// FP8 weights (W8): the e4m3 weight rows go through the LDS ring as bytes
+// and each wave converts its fragments exactly to bf16
+// (v_cvt_scalef32_pk_bf16_fp8) ahead of their MFMAs; the row scale multiplies
+// the accumulators in the epilogue (or the split-K partials).  (Tiles over BK
+// = 32 that are not pipelined load the fragments from global memory.)
 //
 // Split precision: when A_lo is set, the activation is carried as
 // hi + lo bf16 planes (lo = bf16(x - hi)) and every fragment pair issues two
@@ -406,8 +406,8 @@ constexpr bool GemmLnEpilogueOk() {
 
 // fp8 weights (W8): the e4m3 rows go through the LDS ring as bytes (BK
 // codes per row) when a stage's 1 KiB wave-loads split evenly over the
-// waves; otherwise each wave loads its own weight fragments from global
-// memory.
+// waves (every pipelined tile); otherwise each wave loads its own weight
+// fragments from global memory.
 template <int BM, int BN, int BK, int WM, int WN, bool SPLIT>
 constexpr bool W8InLds() {
   return ((SPLIT ? 2 : 1) * BM * BK * 2 + BN * BK) % (1024 * WM * WN) == 0;
@@ -456,7 +456,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t BufferRsrc(const void *base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0x7FFFFFFF, 0x00020000);
 }
 
-template <int BM, int BN, int BK, int ST, int WM, int WN, bool SPLIT, int STAGE>
+template <int BM, int BN, int BK, int ST, int WM, int WN, bool SPLIT, bool W8, int STAGE>
 __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t *lds, int m0,
                                               int n0, int k_begin, int KT,
                                               f32x4 (&acc)[BM / WM / 16][BN / WN / 16]) {
@@ -467,7 +467,8 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
   constexpr int A_ROWS = P * BM;
   constexpr int CPR = BK / 8, RPL = 64 / CPR;  // 16-byte chunks per row, rows per wave-load
   constexpr int LPW = STAGE * 2 / 1024 / NWAVES;
-  static_assert(BM % RPL == 0 && BN % RPL == 0, "a wave-load stays inside one operand");
+  constexpr int W_RPL = W8 ? 2 * RPL : RPL;  // e4m3 weight rows are half as long
+  static_assert(BM % RPL == 0 && BN % W_RPL == 0, "a wave-load stays inside one operand");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / WN, wn = wave % WN;
@@ -480,14 +481,22 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
   // a scalar one.  (The FLAT form, global_load_lds, counts as a possible
   // LDS access for the compiler's wait-count pass, which then waits for
   // every outstanding LDS read, lgkmcnt(0), wherever it waits for one.)
+  // e4m3 weight rows (BK bytes) lie unswizzled: a fragment read covers 16
+  // whole consecutive rows.
   __amdgpu_buffer_rsrc_t rsrc[LPW];
   unsigned goff[LPW];
+  int kstep[LPW];  // bytes per K step
 #pragma unroll
   for (int j = 0; j < LPW; ++j) {
     const int L = wave * LPW + j;
     const int row = L * RPL + lane / CPR;
     const int chunk = (lane % CPR) ^ ((row >> 1) & 3);
-    if (L * RPL < BM) {
+    kstep[j] = W8 && L * RPL >= A_ROWS ? BK : BK * 2;
+    if (W8 && L * RPL >= A_ROWS) {
+      const int off = (L * RPL - A_ROWS) * BK * 2 + lane * 16;
+      rsrc[j] = BufferRsrc(p.W8);
+      goff[j] = static_cast<unsigned>(min(n0 + off / BK, p.N - 1)) * p.ldw + k_begin + off % BK;
+    } else if (L * RPL < BM) {
       rsrc[j] = BufferRsrc(p.A);
       goff[j] = 2u * (static_cast<unsigned>(min(m0 + row, p.M - 1)) * p.lda + k_begin + chunk * 8);
     } else if (SPLIT && L * RPL < 2 * BM) {
@@ -503,7 +512,7 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
   const int ldsw = __builtin_amdgcn_readfirstlane(wave * LPW * 512);  // elements
   auto fill_one = [&](int s, int slot, int j) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc[j], MFH_LDS_PTR(lds + slot * STAGE + ldsw + j * 512),
-                                             16, goff[j], s * (BK * 2), 0, 0);
+                                             16, goff[j], s * kstep[j], 0, 0);
   };
   auto fill = [&](int s, int slot) {
 #pragma unroll
@@ -512,14 +521,17 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
   };
 
   const int a_off = Swz<BK>(wm * (BM / WM) + fr, fc);
-  const int w_off = A_ROWS * BK + Swz<BK>(wn * (BN / WN) + fr, fc);
+  const int w_off = A_ROWS * BK + (W8 ? (wn * (BN / WN) + fr) * (BK / 2) + fc * 4
+                                      : Swz<BK>(wn * (BN / WN) + fr, fc));
   auto read_a = [&](bf16x8 (&a)[TM], const std::uint16_t *base, int q) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
       a[i] = *reinterpret_cast<const bf16x8 *>(base + a_off + (q * BM + i * 16) * BK);
   };
-  auto read_w = [&](bf16x8 &w, const std::uint16_t *base, int j) {
-    w = *reinterpret_cast<const bf16x8 *>(base + w_off + j * 16 * BK);
+  // Weight fragment j: as read (e4m3 codes with W8) and as the MFMAs take it.
+  using WRaw = std::conditional_t<W8, u32x2, bf16x8>;
+  auto read_w = [&](WRaw &w, const std::uint16_t *base, int j) {
+    w = *reinterpret_cast<const WRaw *>(base + w_off + j * 16 * (W8 ? BK / 2 : BK));
   };
   auto mfma_group = [&](const bf16x8 &w, const bf16x8 (&a)[TM], int j) {
 #pragma unroll
@@ -569,7 +581,7 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
     asm volatile("s_barrier" ::: "memory");
   };
 
-  bf16x8 w[TN];
+  WRaw w[TN];
   // Compile-time switches of a step: whether a next stage is read, and
   // whether a later one is loaded.
   using Yes = std::integral_constant<bool, true>;
@@ -604,12 +616,28 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
 #pragma unroll
     for (int j = 0; j < TN; ++j)
       read_w(w[j], lds, j);
+    // e4m3 codes are converted in the hi half, fragment j + 1 while fragment
+    // j's MFMAs run, and kept for the lo half.
+    bf16x8 wb[TN];
+    auto take_w = [&](int j) {
+      if constexpr (W8)
+        wb[j] = Fp8x8ToBf16(w[j]);
+    };
+    auto w_of = [&](int j) -> const bf16x8 & {
+      if constexpr (W8)
+        return wb[j];
+      else
+        return w[j];
+    };
     // hi half of a step whose stage is `cur`: the step's lo fragments are
     // read behind its first MFMA group.
     auto hi_half = [&](auto load, const std::uint16_t *cur, int s, int slot) {
+      take_w(0);
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        mfma_group(w[j], ahi, j);
+        if (j + 1 < TN)
+          take_w(j + 1);
+        mfma_group(w_of(j), ahi, j);
         __builtin_amdgcn_sched_barrier(0);
         if (j == 0)
           read_a(alo, cur, 1);
@@ -625,7 +653,7 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
     auto lo_half = [&](auto more, auto load, const std::uint16_t *nxt, int s, int slot) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        mfma_group(w[j], alo, j);
+        mfma_group(w_of(j), alo, j);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (decltype(more)::value) {
           if (j == 0)
@@ -672,6 +700,12 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
 #pragma unroll
     for (int j = 0; j < TN; ++j)
       read_w(w[j], lds, j);
+    auto w_of = [&](int j) -> bf16x8 {
+      if constexpr (W8)
+        return Fp8x8ToBf16(w[j]);
+      else
+        return w[j];
+    };
     auto rest = [&](auto more, auto load, const std::uint16_t *nxt, int s, int slot) {
       // Nothing is in flight here (the barrier's wait drained the reads);
       // saying so keeps the wait-count pass from draining mid-step.
@@ -684,7 +718,7 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 1; j < TN; ++j) {
-        mfma_group(w[j], a, j);
+        mfma_group(w_of(j), a, j);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (decltype(more)::value)
           read_w(w[j], nxt, j);
@@ -695,11 +729,11 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
 #pragma unroll
         for (int i = 0; i < TM; ++i)
           a[i] = an[i];
-        mfma_group(w[0], a, 0);
+        mfma_group(w_of(0), a, 0);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    mfma_group(w[0], a, 0);
+    mfma_group(w_of(0), a, 0);
     __builtin_amdgcn_sched_barrier(0);
     if (KT > 1)
       sync_first();
@@ -742,7 +776,7 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
 // wave.  The loop is rotated to begin right after the barrier, where no LDS
 // read is in flight.  The loads of a stage are spread over the MFMA groups
 // of an iteration.
-template <int BM, int BN, int ST, int WM, int WN, bool SPLIT, int STAGE>
+template <int BM, int BN, int ST, int WM, int WN, bool SPLIT, bool W8, int STAGE>
 __device__ __forceinline__ void DoubleBufferLoop(const GemmParams &p, std::uint16_t *lds, int m0,
                                                  int n0, int k_begin, int KT,
                                                  f32x4 (&acc)[BM / WM / 16][BN / WN / 16]) {
@@ -751,7 +785,9 @@ __device__ __forceinline__ void DoubleBufferLoop(const GemmParams &p, std::uint1
   constexpr int P = SPLIT ? 2 : 1;
   constexpr int RPL = 8;  // rows of 128 bytes per 1 KiB wave-load
   constexpr int LPW = STAGE * 2 / 1024 / NWAVES;
-  static_assert(BM % (RPL * NWAVES) == 0 && BN % (RPL * NWAVES) == 0,
+  constexpr int W_RPL = W8 ? 2 * RPL : RPL;  // e4m3 weight rows are 64 bytes
+  constexpr int A_LOADS = P * BM / (RPL * NWAVES);  // of a wave's LPW per stage
+  static_assert(BM % (RPL * NWAVES) == 0 && BN % (W_RPL * NWAVES) == 0,
                 "the wave-loads of one index stay inside one operand");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -763,14 +799,20 @@ __device__ __forceinline__ void DoubleBufferLoop(const GemmParams &p, std::uint1
   // belongs in its slot.
   const __amdgpu_buffer_rsrc_t ra = BufferRsrc(p.A);
   const __amdgpu_buffer_rsrc_t ral = BufferRsrc(SPLIT ? p.A_lo : p.A);
-  const __amdgpu_buffer_rsrc_t rw = BufferRsrc(p.W);
+  const __amdgpu_buffer_rsrc_t rw = W8 ? BufferRsrc(p.W8) : BufferRsrc(p.W);
+  // e4m3 weight rows: four 16-byte chunks, XOR-swizzled with the row's bits
+  // 1 and 2 (two rows per 128 bytes), 16 rows per wave-load.
   unsigned goff[LPW];
 #pragma unroll
   for (int j = 0; j < LPW; ++j) {
     const int first = j * NWAVES * RPL;  // row of wave 0's load
     const int row = first + wave * RPL + lane / 8;
     const int chunk = Swz64Chunk(row, lane % 8);
-    if (first < P * BM)
+    if (W8 && j >= A_LOADS) {
+      const int wrow = ((j - A_LOADS) * NWAVES + wave) * W_RPL + lane / 4;
+      goff[j] = static_cast<unsigned>(min(n0 + wrow, p.N - 1)) * p.ldw + k_begin +
+                ((lane % 4) ^ ((wrow >> 1) & 3)) * 16;
+    } else if (first < P * BM)
       goff[j] = 2u * (static_cast<unsigned>(min(m0 + row % BM, p.M - 1)) * p.lda + k_begin +
                       chunk * 8);
     else
@@ -782,23 +824,34 @@ __device__ __forceinline__ void DoubleBufferLoop(const GemmParams &p, std::uint1
     const int first = j * NWAVES * RPL;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         first < BM ? ra : first < P * BM ? ral : rw,
-        MFH_LDS_PTR(lds + slot * STAGE + ldsw + j * NWAVES * 512), 16, goff[j], s * (BK * 2), 0, 0);
+        MFH_LDS_PTR(lds + slot * STAGE + ldsw + j * NWAVES * 512), 16, goff[j],
+        s * (W8 && j >= A_LOADS ? BK : BK * 2), 0, 0);
   };
 
   // Fragment (plane q, row tile i) of substep kk, and weight fragment j.
   // (Rows 16 apart share their swizzle.)
   const int a_row = wm * (BM / WM) + fr, w_row = P * BM + wn * (BN / WN) + fr;
   const int a_off[2] = {Swz<BK>(a_row, fc), Swz<BK>(a_row, 4 + fc)};
-  const int w_off[2] = {Swz<BK>(w_row, fc), Swz<BK>(w_row, 4 + fc)};
+  // (W8: substep kk's eight codes of a row are half fc & 1 of its chunk 2 kk
+  // + fc / 2.)
+  const int w8_row = wn * (BN / WN) + fr;
+  auto w8_off = [&](int kk) {
+    return P * BM * BK + w8_row * (BK / 2) +
+           ((2 * kk + (fc >> 1)) ^ ((w8_row >> 1) & 3)) * 8 + (fc & 1) * 4;
+  };
+  const int w_off[2] = {W8 ? w8_off(0) : Swz<BK>(w_row, fc),
+                        W8 ? w8_off(1) : Swz<BK>(w_row, 4 + fc)};
+  using WRaw = std::conditional_t<W8, u32x2, bf16x8>;
   struct Set {
-    bf16x8 a[P][TM], w[TN];
+    bf16x8 a[P][TM];
+    WRaw w[TN];
   };
   constexpr int kReads = P * TM + TN;
   // Read number r of a set: the weight fragment and hi rows that the first
   // MFMAs take, then the rest.
   auto read_one = [&](Set &f, const std::uint16_t *base, int kk, int r) {
     if (r < TN)
-      f.w[r] = *reinterpret_cast<const bf16x8 *>(base + w_off[kk] + r * 16 * BK);
+      f.w[r] = *reinterpret_cast<const WRaw *>(base + w_off[kk] + r * 16 * (W8 ? BK / 2 : BK));
     else
       f.a[(r - TN) / TM][(r - TN) % TM] = *reinterpret_cast<const bf16x8 *>(
           base + a_off[kk] + ((r - TN) / TM * BM + (r - TN) % TM * 16) * BK);
@@ -816,12 +869,23 @@ __device__ __forceinline__ void DoubleBufferLoop(const GemmParams &p, std::uint1
   // issuing half `h` of the loads of stage s.
   auto substep = [&](const Set &f, auto more, Set &n, const std::uint16_t *base, int kk, auto load,
                      int h, int s, int slot) {
+    // e4m3 codes are converted one fragment ahead of their first MFMAs.
+    bf16x8 wb[TN];
+    auto take_w = [&](int j) {
+      if constexpr (W8)
+        wb[j] = Fp8x8ToBf16(f.w[j]);
+      else
+        wb[j] = f.w[j];
+    };
+    take_w(0);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       const int q = g / TN, j = g % TN;
+      if (g + 1 < TN)
+        take_w(g + 1);
 #pragma unroll
       for (int i = 0; i < TM; ++i)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[j], f.a[q][i], acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[j], f.a[q][i], acc[i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (decltype(more)::value) {
         // All reads within the first three quarters of the groups.
@@ -1012,7 +1076,7 @@ __global__ __launch_bounds__(WM *WN * 64, PIPE && WM * WN == 4 ? 2 : 1) void Gem
   // dimensions halved.
   static_assert(!F8 || (BK == 64 && !SPLIT && !W8), "fp8 activations: BK = 64 bytes pairs");
   static_assert(BK == 32 || BK == 64, "BK is 32 or 64");
-  static_assert(!PIPE || (!W8 && !F8), "pipelined loops: bf16 weights");
+  static_assert(!PIPE || (!F8 && !W8G), "pipelined loops: weights through LDS, bf16 activations");
   static_assert(!LO8 || (PIPE && !SPLIT), "fp8 lo correction follows the single-plane hi pass");
   static_assert(LOADS % NWAVES == 0, "stage loads must split evenly over waves");
   constexpr int LPW = LOADS / NWAVES;
@@ -1054,38 +1118,22 @@ __global__ __launch_bounds__(WM *WN * 64, PIPE && WM * WN == 4 ? 2 : 1) void Gem
   // l / CPR of its wave-load, physical chunk l % CPR, so it fetches the
   // logical chunk that the swizzle puts there.  Rows past M or N read a
   // clamped valid row: they only feed outputs that are never stored.  The
-  // e4m3 weight rows (W8L) are BK bytes, 1024 / BK per wave-load, lane l
-  // fetching the wave-load's l-th 16 bytes unswizzled (a fragment read
-  // covers 16 whole consecutive rows).  kstep: bytes per K step.
-  const char *src[LPW];
-  int kstep[LPW];
+  const std::uint16_t *src[LPW];
   int dst[LPW];
 #pragma unroll
   for (int j = 0; j < LPW; ++j) {
     const int L = wave * LPW + j;
-    if (W8L && L * 1024 >= A_BYTES) {
-      const int off = L * 1024 - A_BYTES + lane * 16;
-      const int row = off / BK;
-      src[j] = reinterpret_cast<const char *>(
-          p.W8 + static_cast<size_t>(min(n0 + row, p.N - 1)) * p.ldw + k_begin + off % BK);
-      kstep[j] = BK;
-    } else {
-      const int row = L * RPL + lane / CPR;
-      const int phys = lane % CPR;
-      const int chunk = BK == 64 ? Swz64Chunk(row, phys) : (phys ^ ((row >> 1) & 3));
-      const std::uint16_t *s16;
-      if (row < BM) {
-        s16 = p.A + static_cast<size_t>(min(m0 + row, p.M - 1)) * p.lda + k_begin + chunk * 8;
-      } else if (SPLIT && row < 2 * BM) {
-        s16 = p.A_lo + static_cast<size_t>(min(m0 + row - BM, p.M - 1)) * p.lda + k_begin +
-              chunk * 8;
-      } else {
-        s16 = p.W + static_cast<size_t>(min(n0 + row - A_ROWS, p.N - 1)) * p.ldw + k_begin +
-              chunk * 8;
-      }
-      src[j] = reinterpret_cast<const char *>(s16);
-      kstep[j] = BK * 2;
-    }
+    const int row = L * RPL + lane / CPR;
+    const int phys = lane % CPR;
+    const int chunk = BK == 64 ? Swz64Chunk(row, phys) : (phys ^ ((row >> 1) & 3));
+    if (row < BM)
+      src[j] = p.A + static_cast<size_t>(min(m0 + row, p.M - 1)) * p.lda + k_begin + chunk * 8;
+    else if (SPLIT && row < 2 * BM)
+      src[j] = p.A_lo + static_cast<size_t>(min(m0 + row - BM, p.M - 1)) * p.lda + k_begin +
+               chunk * 8;
+    else
+      src[j] = p.W + static_cast<size_t>(min(n0 + row - A_ROWS, p.N - 1)) * p.ldw + k_begin +
+               chunk * 8;
     dst[j] = L * 512;
   }
 
@@ -1113,7 +1161,7 @@ __global__ __launch_bounds__(WM *WN * 64, PIPE && WM * WN == 4 ? 2 : 1) void Gem
     if (!PIPE && s < KT) {
 #pragma unroll
       for (int j = 0; j < LPW; ++j)
-        __builtin_amdgcn_global_load_lds(static_cast<const void *>(src[j] + s * kstep[j]),
+        __builtin_amdgcn_global_load_lds(static_cast<const void *>(src[j] + s * BK),
                                          MFH_LDS_PTR(lds + s * STAGE + dst[j]), 16, 0, 0);
     }
 
@@ -1128,9 +1176,9 @@ __global__ __launch_bounds__(WM *WN * 64, PIPE && WM * WN == 4 ? 2 : 1) void Gem
   if constexpr (PIPE) {
 #if defined(__HIP_DEVICE_COMPILE__)
     if constexpr (BK == 64)
-      DoubleBufferLoop<BM, BN, ST, WM, WN, SPLIT, STAGE>(p, lds, m0, n0, k_begin, KT, acc);
+      DoubleBufferLoop<BM, BN, ST, WM, WN, SPLIT, W8, STAGE>(p, lds, m0, n0, k_begin, KT, acc);
     else
-      PipelinedLoop<BM, BN, BK, ST, WM, WN, SPLIT, STAGE>(p, lds, m0, n0, k_begin, KT, acc);
+      PipelinedLoop<BM, BN, BK, ST, WM, WN, SPLIT, W8, STAGE>(p, lds, m0, n0, k_begin, KT, acc);
     if constexpr (LO8)
       Lo8Loop<BM, BN, WM, WN, 2>(p, lds, m0, n0, acc);
 #endif
@@ -1155,7 +1203,7 @@ __global__ __launch_bounds__(WM *WN * 64, PIPE && WM * WN == 4 ? 2 : 1) void Gem
 #pragma unroll
       for (int j = 0; j < LPW; ++j)
         __builtin_amdgcn_global_load_lds(
-            static_cast<const void *>(src[j] + (kt + ST - 1) * kstep[j]),
+            static_cast<const void *>(src[j] + (kt + ST - 1) * BK),
             MFH_LDS_PTR(next + dst[j]), 16, 0, 0);
     }
     const std::uint16_t *sa = lds + slot * STAGE;
@@ -1205,11 +1253,7 @@ __global__ __launch_bounds__(WM *WN * 64, PIPE && WM * WN == 4 ? 2 : 1) void Gem
       bf16x8 af[TM], bw[TN];
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        if constexpr (W8L)
-          bw[j] = Fp8x8ToBf16(*reinterpret_cast<const u32x2 *>(
-              reinterpret_cast<const std::uint8_t *>(sw) + (wn * WTN + j * 16 + fr) * BK +
-              kk * 32 + fc * 8));
-        else if constexpr (W8G)
+        if constexpr (W8G)
           bw[j] = Fp8x8ToBf16(wq[kk][j]);
         else
           bw[j] = *reinterpret_cast<const bf16x8 *>(
@@ -1684,7 +1728,7 @@ hipError_t LaunchW(const GemmParams &p, hipStream_t stream) {
   // beside Q|K|V and at 24-62 positions where its K is not split, and the
   // split 64 x 64 tiles of 24-62 positions), bf16 outputs and the residual
   // mode; the split-K reduce applies it for split consumers.
-  constexpr bool kLn = !W8 && !F8 && (SPLIT || LO8) && (PIPE || (BM == 64 && BN == 64));
+  constexpr bool kLn = !F8 && (SPLIT || LO8) && (PIPE || (BM == 64 && BN == 64));
   if (p.fold_c || p.out_gamma || p.res_stats) {
     if constexpr (kLn) {
       if constexpr (BN >= kLnStatCols)

@@ -1,5 +1,5 @@
 #include "gemm_tiles.h"
 
 namespace mfh {
-MFH_TILES_W8(MFH_TILE_DEFINE)
+MFH_TILES_W8_A(MFH_TILE_DEFINE)
 }  // namespace mfh

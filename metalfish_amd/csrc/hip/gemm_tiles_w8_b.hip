@@ -1,5 +1,5 @@
 #include "gemm_tiles.h"
 
 namespace mfh {
-MFH_TILES_W8_LARGE(MFH_TILE_DEFINE)
+MFH_TILES_W8_B(MFH_TILE_DEFINE)
 }  // namespace mfh

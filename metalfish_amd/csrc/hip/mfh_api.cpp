@@ -530,12 +530,11 @@ int Infer(const mfh_net_desc &desc, Loader &ld, Dims &d) {
   d.split = desc.precision == MFH_PRECISION_BF16X2 ||
             desc.precision == MFH_PRECISION_BF16X2_GEMM || d.lo8;
   d.split_attn = desc.precision == MFH_PRECISION_BF16X2 || d.lo8;
-  // Measured at the BT4 shape: the panel wins with e4m3 weights (half the
-  // weight bytes to stream; batch 1024 22.29k against 22.09k positions/s
-  // for the tiled GEMM + LayerNorm, batch 256 even), the tiled GEMM +
-  // LayerNorm kernel with bf16.  The panel has no fp8 lo correction:
-  // BF16X2_FP8LO keeps the tiled GEMM.
-  d.fused_ln = !d.lo8 && (desc.fused_layernorm != 0 || desc.weights_dtype == MFH_WEIGHTS_FP8);
+  // The panel only when asked for: since the e4m3 rows too run on the
+  // pipelined tiles with the LayerNorms folded, batch 1024 takes 38.6 ms
+  // against 44.6 with the panel (BF16X2; the panel had won over the
+  // lock-step e4m3 tiles).  The panel has no fp8 lo correction.
+  d.fused_ln = !d.lo8 && desc.fused_layernorm != 0;
   d.wdl = desc.value == MFH_VALUE_WDL;
   d.mlh = desc.moves_left == 1;
   d.act_default = desc.default_activation == MFH_DEFAULT_ACTIVATION_MISH ? mfh::ACT_MISH
@@ -1497,11 +1496,8 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
   auto residual_ln = [&](const std::string &a, int k, const size_t (&w_off)[2],
                          const float *bias, const char *role, float alpha, float eps,
                          const float *g, const float *b, float *y32, bool f8 = false) -> int {
-    // fused_layernorm (default with fp8 weights).  The panel streams each
-    // weight row from L2 for only 64 activation rows, which needs every
-    // weight fragment to feed two MFMAs (split activations); with bf16
-    // weights the tiled GEMM's staged epilogue plus the LayerNorm kernel
-    // measured faster on the BT4 shape.
+    // fused_layernorm: the panel streams each weight row from L2 for only 64
+    // activation rows.
     if (d.fused_ln && d.split && M >= kPanelMinRows &&
         mfh::PanelGemmShapeOk(mfh::PANEL_OUT_LN, E, k)) {
       mfh::PanelGemmParams pp;

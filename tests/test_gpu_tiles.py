@@ -50,8 +50,9 @@ def test_large_tiles_equal_small_ones(m, n, k, act):
         assert (np.abs(small - z) <= bound).all()
 
 
+@pytest.mark.parametrize("weights_dtype", ["bf16", "fp8"])
 @pytest.mark.parametrize("precision", ["bf16x2", "bf16x2_gemm", "bf16"])
-def test_batches_across_tile_rules_agree(precision):
+def test_batches_across_tile_rules_agree(precision, weights_dtype):
     """Two BT4-width layers: batches at the first folded one (24), odd ones,
     one past a tile's whole rounds (65, 129, 257: the rows split over two
     launches) and others agree with batch 4 position by position.  In bf16x2
@@ -63,13 +64,15 @@ def test_batches_across_tile_rules_agree(precision):
     spec = dataclasses.replace(synth.SPECS["bt4"], name="two", layers=2)
     weights = synth.make_weights(spec, seed=2)
     planes, _ = synth.playout_positions(4, seed=9)
-    net = backend.create_network(spec, weights, max_batch=321, device=0, precision=precision)
+    net = backend.create_network(spec, weights, max_batch=321, device=0, precision=precision,
+                                 weights_dtype=weights_dtype)
     small = net.evaluate_batch(planes)
+    assert weights_dtype == "bf16" or "e4m3" in net.info()
     for batch in (24, 25, 33, 43, 64, 65, 100, 129, 200, 257, 300, 321):
         idx = np.arange(batch) % 4
         out = net.evaluate_batch(planes[idx])
         err = np.abs(out["policy"] - small["policy"][idx]).max()
         werr = np.abs(out["wdl"] - small["wdl"][idx]).max()
-        print(f"{precision} batch {batch}: policy {err:.2e} wdl {werr:.2e}", flush=True)
+        print(f"{precision}/{weights_dtype} batch {batch}: policy {err:.2e} wdl {werr:.2e}", flush=True)
         assert err <= tol and werr <= tol
     net.close()
