@@ -32,7 +32,7 @@ HIP_SOURCES = ["hip/gemm_tiles_pipe_a.hip", "hip/gemm_tiles_pipe_b.hip",
                "hip/policy.hip",
                "hip/mfh_api.cpp", "host/policy_tables.cpp"]
 # Host-only parts of libmfhip.so (no device code), compiled with g++.
-HIP_HOST_SOURCES = ["host/weights_file.cpp"]
+HIP_HOST_SOURCES = ["host/weights_file.cpp", "host/pack_planes.cpp"]
 HOST_SOURCES = ["host/chess.cpp", "host/policy_tables.cpp", "host/synth_api.cpp"]
 
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -31,6 +31,7 @@
 #include <stdexcept>
 #include <vector>
 
+#include "../host/pack_planes.h"
 #include "../host/policy_tables.h"
 #include "../host/weights_file.h"
 #include "mfh_kernels.h"
@@ -2108,33 +2109,6 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
   return MFH_OK;
 }
 
-void PackPlanes(const float *planes, int batch, std::uint64_t *masks, float *values) {
-  // PackInputPlanesRaw (reference src/nn/input_plane_packing.h:30-83).
-  for (int b = 0; b < batch; ++b)
-    for (int p = 0; p < kPlanes; ++p) {
-      const float *plane = planes + (static_cast<size_t>(b) * kPlanes + p) * kSquares;
-      const size_t idx = static_cast<size_t>(b) * kPlanes + p;
-      const bool uniform = (p < 104 && p % 13 == 12) || p == 106 || p == 107 || p >= 109;
-      if (uniform) {
-        values[idx] = plane[0];
-        masks[idx] = plane[0] != 0.0f ? ~0ULL : 0ULL;
-        continue;
-      }
-      std::uint64_t mask = 0;
-      float value = 0.0f;
-      for (int sq = 0; sq < kSquares; ++sq) {
-        const float v = plane[sq];
-        if (v != 0.0f) {
-          if (mask == 0)
-            value = v;
-          mask |= 1ULL << sq;
-        }
-      }
-      masks[idx] = mask;
-      values[idx] = value;
-    }
-}
-
 int CheckBatch(const mfh_net *net, int batch) {
   if (!net)
     return SetError(MFH_ERR_INVALID, "null net");
@@ -2556,7 +2530,7 @@ int mfh_net_eval_planes(mfh_net *net, int batch, const float *planes, float *pol
   if (rc != MFH_OK)
     return rc;
   std::lock_guard<std::mutex> lock(net->mu);
-  PackPlanes(planes, batch, reinterpret_cast<std::uint64_t *>(net->pin_in),
+  mfh::PackPlanes(planes, batch, reinterpret_cast<std::uint64_t *>(net->pin_in),
              reinterpret_cast<float *>(net->pin_in +
                                        static_cast<size_t>(net->max_batch) * kPlanes * 8));
   rc = RunStaged(net, batch);
@@ -2930,7 +2904,7 @@ int mfh_net_profile(mfh_net *net, mfh_profile_entry *out, int capacity, int *cou
 int mfh_pack_planes(int batch, const float *planes, uint64_t *masks, float *values) {
   if (batch < 0 || (batch > 0 && (!planes || !masks || !values)))
     return SetError(MFH_ERR_INVALID, "mfh_pack_planes: bad arguments");
-  PackPlanes(planes, batch, masks, values);
+  mfh::PackPlanes(planes, batch, masks, values);
   return MFH_OK;
 }
 
