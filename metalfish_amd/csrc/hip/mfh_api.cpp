@@ -102,6 +102,9 @@ constexpr int kSmolgenFewRowMaxBatch = 16;
 // -> 2.59, 20 2.31 -> 2.29; with the few-row chain at 16 positions it was
 // slower, 2.07 -> 2.19).
 constexpr int kSmolgenSideRows = 1088;
+// Token rows below which dense2's LayerNorm and the global projection are one
+// launch: under 48 positions (measured beside smolgen_bias.hip).
+constexpr int kSmolgenBiasRows = 48 * kSquares;
 
 // BF16X2_FP8LO: the fp8 lo correction runs from this many token rows (128
 // positions); below, the forward is the BF16X2 one.
@@ -1609,6 +1612,17 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
                              B <= kSmolgenFewRowMaxBatch && !net->fp8 &&
                              mfh::SkinnyShapeOk(B, d.Hs, kSquares * d.C) &&
                              mfh::SkinnyShapeOk(B, d.HG, d.Hs);
+  // Dense2's LayerNorm and the global projection in one launch.
+  const bool smolgen_bias =
+      d.smolgen && !d.fused_bias && M < kSmolgenBiasRows && mfh::SmolgenBiasOk(d.H, d.G, kSquares * kSquares);
+  auto run_bias = [&](const mfh::SmolgenBiasParams &p, hipStream_t s) {
+    const double rows = static_cast<double>(p.batch) * p.heads;
+    const double out_bytes = p.out_lo8 ? 3.0 : p.split ? 4.0 : 2.0;
+    StageTimer t(net, s, "gemm_bf16:smolgen_global",
+                 2.0 * rows * p.N * p.gen,
+                 rows * (4.0 * p.gen + out_bytes * p.N) + (p.W8 ? 1.0 : 2.0) * p.N * p.gen);
+    return mfh::LaunchSmolgenBias(p, s, &err_);
+  };
   auto run_sk = [&](const mfh::SkinnyParams &p, const char *role, hipStream_t on = nullptr) {
     const double flops = 2.0 * p.M * p.N * p.K;
     const double bytes = 2.0 * p.N * p.K + 4.0 * p.M * p.K + 4.0 * p.M * p.N;
@@ -1822,21 +1836,48 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
         q.small_lds = share_cus;
         return q;
       };
-      // The shared global projection of the normalised dense2 rows into the
-      // attention bias (unless attention projects the gen vectors itself).
+      // Dense2's LayerNorm and the shared global projection of its rows into
+      // the attention bias: one launch (smolgen_bias.hip) where the shapes
+      // allow, else the LayerNorm, then the projection as a GEMM (unless
+      // attention projects the gen vectors itself).
       auto smolgen_global = [&](hipStream_t s) -> int {
+        // BF16X2_FP8LO: the bias as bf16 hi plus the e4m3 codes of its lo
+        // parts (3 bytes instead of fp32's 4, written here and read by
+        // attention).
+        std::uint8_t *codes = qkv_codes ? ws.S<std::uint8_t>("bias_lo8") : nullptr;
+        if (smolgen_bias) {
+          mfh::SmolgenBiasParams pb;
+          pb.x = sg2;
+          pb.gamma = net->W<float>(L.sg_ln2_g);
+          pb.beta = net->W<float>(L.sg_ln2_b);
+          pb.batch = B;
+          pb.heads = d.H;
+          pb.gen = d.G;
+          if (net->fp8) {
+            pb.W8 = net->W<std::uint8_t>(net->global_w[0]);
+            pb.wscale = net->W<float>(net->global_w[1]);
+          } else {
+            pb.W = net->W<std::uint16_t>(net->global_w[0]);
+          }
+          pb.N = kSquares * kSquares;
+          pb.split = d.split_attn;
+          pb.out = ws.S<void>("bias");
+          pb.out_lo8 = codes;
+          MFH_RUN(run_bias(pb, s));
+          return MFH_OK;
+        }
+        MFH_RUN(run_ln(ln(sg2, B, d.HG, 1e-3f, net->W<float>(L.sg_ln2_g),
+                          net->W<float>(L.sg_ln2_b), nullptr, "sg2n"),
+                       s));
         if (d.fused_bias)
           return MFH_OK;
         mfh::GemmParams pg = chain_gemm("sg2n", d.G, net->global_w, d.G, B * d.H,
                                         kSquares * kSquares, d.G, nullptr,
                                         d.split_attn ? mfh::GEMM_OUT_F32 : mfh::GEMM_OUT_BF16,
                                         ws.S<void>("bias"), nullptr, kSquares * kSquares);
-        if (qkv_codes) {
-          // BF16X2_FP8LO: the bias as bf16 hi plus the e4m3 codes of its lo
-          // parts (3 bytes instead of fp32's 4, written here and read by
-          // attention).
+        if (codes) {
           pg.out_mode = mfh::GEMM_OUT_BF16;
-          pg.C_lo8 = ws.S<std::uint8_t>("bias_lo8");
+          pg.C_lo8 = codes;
           pg.ldc8 = kSquares * kSquares;
         }
         MFH_RUN(run(pg, "smolgen_global", s));
@@ -1861,9 +1902,6 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
       }
       if (few_row_dense) {
         MFH_RC(smolgen_dense_few_row(L, on, false));
-        MFH_RUN(run_ln(ln(sg2, B, d.HG, 1e-3f, net->W<float>(L.sg_ln2_g),
-                          net->W<float>(L.sg_ln2_b), nullptr, "sg2n"),
-                       on));
         return smolgen_global(on);
       }
       const int flat = kSquares * d.C;
@@ -1890,9 +1928,6 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
       p2.act = d.act_smolgen;
       p2.partials = nullptr;  // no automatic split-K
       MFH_RUN(run(p2, "smolgen_dense2", on));
-      MFH_RUN(run_ln(ln(sg2, B, d.HG, 1e-3f, net->W<float>(L.sg_ln2_g),
-                        net->W<float>(L.sg_ln2_b), nullptr, "sg2n"),
-                     on));
       return smolgen_global(on);
     };
     if (L.smolgen && !d.fused_bias) {

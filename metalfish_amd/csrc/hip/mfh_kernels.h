@@ -384,6 +384,32 @@ constexpr int SmolgenBiasIndex(int query, int key) {
          (key & 3);
 }
 
+// The smolgen chain's last LayerNorm and the shared global projection in one
+// launch: rows x [batch][heads * gen] fp32 (dense2's activated output),
+// out[batch * heads][N] = LN(x)[b][h segment] . W[N][gen]^T, the LayerNorm
+// over the whole heads * gen row.  `split`: the normalised rows as bf16 hi +
+// lo, fp32 output, or with out_lo8 bf16 plus e4m3 codes of the lo parts;
+// otherwise single bf16 rows and output.
+struct SmolgenBiasParams {
+  const float *x = nullptr;
+  const float *gamma = nullptr, *beta = nullptr;
+  float eps = 1e-3f;
+  int batch = 0, heads = 0, gen = 0;
+  const std::uint16_t *W = nullptr;
+  const std::uint8_t *W8 = nullptr;  // e4m3 codes with row scales instead
+  const float *wscale = nullptr;
+  int N = 0;
+  bool split = false;
+  void *out = nullptr;
+  std::uint8_t *out_lo8 = nullptr;
+  // Set by LaunchSmolgenBias: positions and column tiles per workgroup,
+  // 16-bit reciprocal of a position's 256-element chunks.
+  int positions = 0, tiles = 0, chunk_inv = 0;
+};
+// Whether LaunchSmolgenBias takes these shapes.
+bool SmolgenBiasOk(int heads, int gen, int n);
+hipError_t LaunchSmolgenBias(const SmolgenBiasParams &p, hipStream_t stream, std::string *err);
+
 struct AttentionParams {
   const std::uint16_t *qkv = nullptr;
   const std::uint16_t *qkv_lo = nullptr;
