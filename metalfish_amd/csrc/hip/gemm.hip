@@ -92,6 +92,10 @@ bool Aligned(const void *ptr, std::uintptr_t bytes) {
 // Rows from which the tile rules for large problems apply (below them,
 // 64 x 64 tiles over the whole K or split-K).
 constexpr int kLargeRows = 1536;
+// Rows from which the time model below is fitted for a long K (LaunchGemm).
+// With bf16 weights up to 16 positions: at 17 to 23, beside the smolgen chain,
+// it moved the forward by -0.4 to +0.7 %; with e4m3 weights 20 gained 1.8 %.
+constexpr int kModelRows = 256, kModelRowsEnd = 1088;
 
 // 256 x 256 tiles where they fill whole rounds of 256 workgroups (bf16
 // activations, one K slice, from the large-problem rows).
@@ -119,6 +123,7 @@ enum class Tile {
   kWide,     // 128 x 256, four waves, two stages of 32 KiB (beside the chain)
   k128,      // 128 x 128 over BK = 64, three stages of 48 KiB
   k64x128,   // 64 x 128 over BK = 64, four stages of 32 KiB
+  k64Three,  // 64 x 64 over BK = 64, three stages of 24 KiB (two per CU)
   k64,       // 64 x 64 over BK = 64, two stages of 24 KiB (three per CU)
   kNarrow,   // 64 x 64 over BK = 32, two stages (narrow N, beside the chain)
   kSplitK,   // split over K, the reduce kernel applying the LayerNorm
@@ -155,7 +160,7 @@ constexpr TileTime kOneTimes[] = {
     {Tile::kOne256x128, 256, 128, 256, 5.f, 2.f, 2.5f, 9.6f, 5.4f},
     {Tile::kOne128, 128, 128, 256, 2.f, 0.5f, 1.f, 6.f, 3.f},
     {Tile::kOne128Two, 128, 128, 512, 2.f, 0.5f, 0.f, 10.5f, 11.f},
-    {Tile::kOne64x128, 64, 128, 512, 1.5f, 0.5f, 0.f, 1.6f, 10.f},
+    {Tile::kOne64x128, 64, 128, 512, 1.5f, 0.5f, 0.f, 4.f, 7.f},
     {Tile::kOne64, 64, 64, 768, 1.5f, 0.5f, 0.f, 2.1f, 6.4f},
 };
 constexpr TileTime kTileTimes[] = {
@@ -164,6 +169,7 @@ constexpr TileTime kTileTimes[] = {
     {Tile::k128, 128, 128, 256, 2.5f, 1.5f, 1.f, 9.5f, 5.f},
     {Tile::k64x128, 64, 128, 256, 1.5f, 1.f, 0.5f, 5.8f, 2.5f},
     {Tile::k64, 64, 64, 768, 2.f, 1.f, 0.f, 6.f, 6.5f},
+    {Tile::k64Three, 64, 64, 256, 0.5f, 1.f, 0.f, 3.3f, 1.9f},
 };
 
 float LaunchTime(const TileTime &t, int M, const GemmParams &p) {
@@ -204,12 +210,24 @@ Tile BestTile(const GemmParams &p, int M, float *us) {
   return best;
 }
 
+// A short K under a wide output (the smolgen global projection): the time
+// goes into the stores, which two workgroups per CU overlap with each
+// other's loads.  N = 4096, K = 256, split with fp32 output: 8192 rows 47.6
+// us (256 x 256 tiles 53.1), 9600 59.1 (71.7), 16384 106 (112), but 2048
+// 17.8 (128 x 256 with eight waves 17.2); single bf16 8192 rows 30.2 (256 x 256 34.3),
+// 9600 35.7 (256 x 128 39.7), 16384 56.3 (60.7), 32768 131 (122.9).  Past 16384
+// rows the 256 x 256 tiles' rounds are long enough (batch 1024 0.6 % slower).
+bool StoreBound(const GemmParams &p) {
+  return p.K <= 256 && p.M > 2048 && p.M <= 16384 && p.N >= 2048 && p.N % 256 == 0 && p.act == ACT_NONE && !p.beside_chain &&
+         p.out_mode != GEMM_OUT_RESID_F32 && !p.fold_c;
+}
+
 // Rows of p to run on whole rounds of 256 x 256 tiles, the rest following as
 // a launch of its own on smaller ones (0: one launch).  A last round that is
 // nearly empty costs as much as a full one: out-projection at 19200 rows
 // (300 tiles of 256 x 256) 129 us on them, 100 on 128 x 128, 67 + 20 split.
 int RowsFirst(const GemmParams &p) {
-  if (p.N % 256 || p.beside_chain || p.M < kLargeRows)
+  if (p.N % 256 || p.beside_chain || p.M < kLargeRows || StoreBound(p))
     return 0;
   const TileTime &whole = p.A_lo ? kTileTimes[0] : kOneTimes[0];
   const int nbn = p.N / 256, nbm = p.M / 256;
@@ -237,6 +255,8 @@ Tile LargeTile(const GemmParams &p) {
   if (!p.A_lo) {
     if (ln || p.M < kLargeRows || p.N < 128)
       return Tile::kNone;
+    if (StoreBound(p))
+      return Tile::kOne128Two;
     if (p.beside_chain)
       return GemmWholeRoundTiles(p) ? Tile::kOne256 : p.W8 ? Tile::kOne128Two : Tile::kOneSlim;
     float us;
@@ -262,6 +282,8 @@ Tile LargeTile(const GemmParams &p) {
       return Tile::k256Two;
     return !ln || p.N % 256 == 0 ? Tile::kWide : Tile::kNone;
   }
+  if (StoreBound(p))
+    return Tile::kWide;
   float us;
   return BestTile(p, p.M, &us);
 }
@@ -311,6 +333,8 @@ hipError_t LaunchTile(Tile t, const GemmParams &p, hipStream_t stream) {
     return LaunchPipe<64, 128, 64, 4, 2, 4, true>(p, stream);
   case Tile::k64:
     return LaunchPipe<64, 64, 64, 2, 2, 2, true>(p, stream);
+  case Tile::k64Three:
+    return LaunchPipe<64, 64, 64, 3, 2, 2, true>(p, stream);
   case Tile::kNarrow:
     return LaunchStep32<true>(p, stream);
   case Tile::kOne256:
@@ -558,9 +582,20 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
   if (f8)
     return big_tiles % 256 == 0 ? LaunchW<256, 256, 64, 2, 4, 2, false, false, true>(p, stream)
                                 : LaunchW<128, 128, 64, 2, 2, 4, false, false, true>(p, stream);
-  // 64 x 64 tiles over the whole K (Q|K|V at 4-31 positions, the
-  // out-projection and FFN at 16-31, the smolgen dense2 and global
-  // projection at some batches): from 256 rows up, or over K >= 1024, a
+  // Q|K|V, out-projection and FFN over the whole K at 4 to 23 positions: the
+  // tile by the time model, as for the large shapes.  Measured alone against
+  // the 64 x 64 tiles below, split: Q|K|V (N = 3136) at 512 rows 10.9 us on 64
+  // x 128 (12.5), 768 17.5 on two-stage 64 x 64 (18.9), 1024 18.8 on 128 x 128
+  // (21.8); FFN1 at 768 11.1 on 64 x 128 (12.4); single bf16 Q|K|V at 1024 12.4
+  // on 128 x 128 (16.5).  (Beside the chain, from 17 positions, the 128 x 128
+  // tiles' 144 KiB keep its workgroups off the CU: batch 20 4 % slower.)
+  if (p.M >= kModelRows && p.M < (p.W8 ? kLargeRows : kModelRowsEnd) && p.N >= 128 && p.k_splits == 1 && p.K % 64 == 0 &&
+      p.K >= 512 && !p.small_lds && !p.beside_chain) {
+    float us;
+    return LaunchTile(BestTile(p, p.M, &us), p, stream);
+  }
+  // 64 x 64 tiles over the whole K otherwise (the smolgen dense2 and other
+  // short K, few rows or columns): from 256 rows up, or over K >= 1024, a
   // three-stage ring keeps two K steps in flight (batch 16 forward 2.30 ->
   // 2.05 ms, batch 8 1.75 -> 1.68, batch 256 +0.9 %, batch 3 1.51 -> 1.36;
   // Q|K|V took 16.0 us at 192 rows with two stages, 11.6 us at 256 rows

@@ -1,4 +1,4 @@
-"""The GEMM tiles of the large shapes (from 1536 rows): every tile gives the
+"""The GEMM tiles of the larger shapes (from 256 rows): every tile gives the
 bits of the 64 x 64 tiles that small shapes take, and forwards at batches
 where the choice of tile, a row split or the LayerNorm fold changes agree
 with small batches."""
@@ -24,7 +24,9 @@ def _bits(rng, shape, scale=1.0):
 @pytest.mark.parametrize("m,n,k", [(1536, 128, 64), (1537, 130, 128), (1600, 1024, 320),
                                    (2047, 1024, 1024), (4096, 1024, 1024), (4100, 1536, 1024),
                                    (6400, 1024, 1536), (12800, 256, 192), (16385, 256, 64),
-                                   (16640, 1024, 256), (1536, 1056, 96)])
+                                   (16640, 1024, 256), (1536, 1056, 96), (2048, 2048, 256),
+                                   (1601, 2304, 128), (256, 1536, 1024), (511, 3136, 1024),
+                                   (700, 1538, 512), (1030, 3136, 1024), (1535, 1536, 640)])
 @pytest.mark.parametrize("act", ["none", "mish"])
 def test_large_tiles_equal_small_ones(m, n, k, act):
     """The MFMAs of an output accumulate over K in one order on every tile,
@@ -53,7 +55,8 @@ def test_large_tiles_equal_small_ones(m, n, k, act):
 @pytest.mark.parametrize("weights_dtype", ["bf16", "fp8"])
 @pytest.mark.parametrize("precision", ["bf16x2", "bf16x2_gemm", "bf16"])
 def test_batches_across_tile_rules_agree(precision, weights_dtype):
-    """Two BT4-width layers: batches at the first folded one (24), odd ones,
+    """Two BT4-width layers: batches below the fold whose tiles differ (8 to
+    20), the first folded one (24), odd ones,
     one past a tile's whole rounds (65, 129, 257: the rows split over two
     launches) and others agree with batch 4 position by position.  In bf16x2
     to summation-order noise, 1e-4, as between any two batch sizes; the
@@ -68,7 +71,7 @@ def test_batches_across_tile_rules_agree(precision, weights_dtype):
                                  weights_dtype=weights_dtype)
     small = net.evaluate_batch(planes)
     assert weights_dtype == "bf16" or "e4m3" in net.info()
-    for batch in (24, 25, 33, 43, 64, 65, 100, 129, 200, 257, 300, 321):
+    for batch in (8, 12, 16, 20, 24, 25, 33, 43, 64, 65, 100, 129, 200, 257, 300, 321):
         idx = np.arange(batch) % 4
         out = net.evaluate_batch(planes[idx])
         err = np.abs(out["policy"] - small["policy"][idx]).max()
