@@ -70,6 +70,144 @@ hipError_t Reduce(const GemmParams &p, const float *part, int splits, hipStream_
   return LaunchReduce<GEMM_OUT_BF16, ACT_RUNTIME>(p, part, splits, stream);
 }
 
+// Narrow outputs (the smolgen compression: 32 columns, K = 1024) at many
+// rows.  There is no reuse to stage for: a workgroup takes 32 rows x 32
+// columns, its eight waves an eighth of K each, straight from memory into
+// registers with every load of 128 K elements in flight at once, and the
+// partial tiles are summed in wave order through LDS before the epilogue.
+// What bounds it: the rows' bytes at large batches, the launch and one
+// latency at small ones; the ring of 64 x 64 tiles that it replaces had 16 to
+// 32 latencies in a row on too few workgroups, or a split over K with a
+// second launch to sum it.
+constexpr int kNarrowWaves = 8, kNarrowTile = 32;
+template <bool SPLIT, bool W8, bool LN>
+__global__ __launch_bounds__(kNarrowWaves * 64, 2) void NarrowKernel(GemmParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int P = SPLIT ? 2 : 1, PITCH = kNarrowTile + 4;
+  __shared__ float red[kNarrowWaves][kNarrowTile][PITCH];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int fr = lane & 15, fc = lane >> 4;
+  const int m0 = blockIdx.x * kNarrowTile, n0 = blockIdx.y * kNarrowTile;
+  const int ks = p.K / kNarrowWaves, first = wave * ks;
+  const std::uint16_t *ar[P][2];
+  size_t wr[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    // (Rows and columns past the edge repeat the last one.)
+    const size_t row = min(m0 + i * 16 + fr, p.M - 1), col = min(n0 + i * 16 + fr, p.N - 1);
+    ar[0][i] = p.A + row * p.lda + first + fc * 8;
+    if constexpr (SPLIT)
+      ar[1][i] = p.A_lo + row * p.lda + first + fc * 8;
+    wr[i] = col * p.ldw + first + fc * 8;
+  }
+  // The epilogue's operands, asked for with the first rows: a thread of the
+  // first four waves ends up with four outputs of row r.
+  const int r = threadIdx.x / 8, c = threadIdx.x % 8 * 4;
+  const bool out = r < kNarrowTile && m0 + r < p.M && n0 + c < p.N;
+  float b[4] = {}, mu = 0.f, rs = 1.f, fold[4] = {}, scale[4] = {1.f, 1.f, 1.f, 1.f};
+  using WRaw = std::conditional_t<W8, u32x2, bf16x8>;
+  f32x4 acc[2][2] = {};
+  for (int k = 0; k < ks; k += 128) {
+    bf16x8 a[4][P][2];
+    WRaw w[4][2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (k + 32 * t < ks)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+          for (int q = 0; q < P; ++q)
+            a[t][q][i] = *reinterpret_cast<const bf16x8 *>(ar[q][i] + k + 32 * t);
+          if constexpr (W8)
+            w[t][i] = *reinterpret_cast<const WRaw *>(p.W8 + wr[i] + k + 32 * t);
+          else
+            w[t][i] = *reinterpret_cast<const WRaw *>(p.W + wr[i] + k + 32 * t);
+        }
+    if (k == 0 && out) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int col = n0 + c + e;  // (N is a multiple of 4)
+        b[e] = p.bias ? p.bias[col] : 0.f;
+        scale[e] = p.wscale ? p.wscale[col] : 1.f;
+        if constexpr (LN)
+          fold[e] = p.fold_c[col];
+      }
+      if constexpr (LN)
+        RowLnStats(p.ln_stats, p.ln_width, p.ln_eps, m0 + r, mu, rs);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (k + 32 * t < ks) {
+        bf16x8 wb[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          if constexpr (W8)
+            wb[j] = Fp8x8ToBf16(w[t][j]);
+          else
+            wb[j] = w[t][j];
+        }
+#pragma unroll
+        for (int q = 0; q < P; ++q)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[j], a[t][q][i], acc[i][j],
+                                                                  0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      *reinterpret_cast<f32x4 *>(&red[wave][i * 16 + fr][j * 16 + fc * 4]) = acc[i][j];
+  __syncthreads();
+  if (!out)
+    return;
+  f32x4 sum = *reinterpret_cast<const f32x4 *>(&red[0][r][c]);
+#pragma unroll
+  for (int v = 1; v < kNarrowWaves; ++v)
+    sum += *reinterpret_cast<const f32x4 *>(&red[v][r][c]);
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    sum[e] = rs * (sum[e] * scale[e] - mu * fold[e]);
+  GemmParams q = p;
+  q.wscale = nullptr;
+  Epilogue4<GEMM_OUT_BF16, ACT_NONE, false>(q, m0 + r, n0 + c, sum, b);
+#endif
+}
+
+template <bool SPLIT, bool W8>
+hipError_t LaunchNarrowW(const GemmParams &p, hipStream_t stream) {
+  const dim3 grid((p.M + kNarrowTile - 1) / kNarrowTile, (p.N + kNarrowTile - 1) / kNarrowTile);
+  if (p.fold_c)
+    hipLaunchKernelGGL((NarrowKernel<SPLIT, W8, true>), grid, dim3(kNarrowWaves * 64), 0, stream,
+                       p);
+  else
+    hipLaunchKernelGGL((NarrowKernel<SPLIT, W8, false>), grid, dim3(kNarrowWaves * 64), 0, stream,
+                       p);
+  return hipGetLastError();
+}
+
+// From 17 positions, where the compression is a launch of its own, to 47: the
+// forward at batch 17 2002 -> 1971 us, 24 2038 -> 1996, 32 2192 -> 2166, 45
+// 2701 -> 2680, bf16 at 32 2001 -> 1953.  Past that its waves and the loads
+// of the same weights by every 32 rows hold up Q|K|V beside it: 48 2 %
+// slower, 128 2.4 %, 300 2 %.
+constexpr int kNarrowRows = 1088, kNarrowRowsEnd = 3072;
+bool NarrowOk(const GemmParams &p) {
+  return p.M >= kNarrowRows && p.M < kNarrowRowsEnd && p.N < 128 && p.N % 4 == 0 && p.K % (32 * kNarrowWaves) == 0 &&
+         p.k_splits == 1 && p.out_mode == GEMM_OUT_BF16 && p.act == ACT_NONE && !p.A8 &&
+         !p.A_lo8 && !p.C_lo8 && p.split_n >= p.N;
+}
+
+hipError_t LaunchNarrow(const GemmParams &p, hipStream_t stream) {
+  if (p.A_lo)
+    return p.W8 ? LaunchNarrowW<true, true>(p, stream) : LaunchNarrowW<true, false>(p, stream);
+  return p.W8 ? LaunchNarrowW<false, true>(p, stream) : LaunchNarrowW<false, false>(p, stream);
+}
+
 // A tile with bf16 or fp8 weights on the pipelined loops.
 template <int BM, int BN, int BK, int ST, int WM, int WN, bool SPLIT>
 hipError_t LaunchPipe(const GemmParams &p, hipStream_t stream) {
@@ -523,6 +661,8 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
   // Large shapes and any folded LayerNorm: the tiles of LargeTile.  (BF16X2_FP8LO: 256 x 256 tiles of
   // eight waves, the hi pass on the four-stage single-bf16 pipelined ring,
   // 128 KiB, then the lo pass on two 64 KiB stages of code rows.)
+  if (NarrowOk(p))
+    return LaunchNarrow(p, stream);
   const Tile tile = LargeTile(p);
   if (tile == Tile::kSplitK) {
     if (!Aligned(p.partials, 16) || !p.vec || p.N % 4)

@@ -79,3 +79,31 @@ def test_batches_across_tile_rules_agree(precision, weights_dtype):
         print(f"{precision}/{weights_dtype} batch {batch}: policy {err:.2e} wdl {werr:.2e}", flush=True)
         assert err <= tol and werr <= tol
     net.close()
+
+
+@pytest.mark.parametrize("compress", [8, 40, 104])
+@pytest.mark.parametrize("precision,weights_dtype", [("bf16x2", "bf16"), ("bf16x2", "fp8"),
+                                                     ("bf16", "bf16"), ("bf16", "fp8")])
+@pytest.mark.parametrize("embedding", [256, 768])
+def test_narrow_products_agree(precision, weights_dtype, compress, embedding):
+    """The compression as a launch of its own on narrow tiles (17 to 47
+    positions; columns of a part of a tile, of two and of four; folded
+    LayerNorm from 24; an eighth of K of 32 and of 96) against batch 4, where
+    it is part of Q|K|V.  Tolerances as between any two batch sizes."""
+    tol = {"bf16x2": 1e-4, "bf16": 3e-2}[precision]
+    spec = dataclasses.replace(synth.SPECS["bt4"], name="narrow", layers=2, embedding=embedding,
+                               heads=embedding // 32, ffn=512, input_ffn=512,
+                               smolgen_compress=compress, smolgen_hidden=64, smolgen_gen=64)
+    weights = synth.make_weights(spec, seed=6, fp8=weights_dtype == "fp8")
+    planes, _ = synth.playout_positions(4, seed=5)
+    net = backend.create_network(spec, weights, max_batch=48, device=0, precision=precision,
+                                 weights_dtype=weights_dtype)
+    small = net.evaluate_batch(planes)
+    for batch in (17, 23, 24, 47, 48):
+        idx = np.arange(batch) % 4
+        out = net.evaluate_batch(planes[idx])
+        err = max(np.abs(out[k] - small[k][idx]).max() for k in ("policy", "wdl"))
+        print(f"{precision}/{weights_dtype} {embedding} x {compress} batch {batch}: {err:.2e}",
+              flush=True)
+        assert err <= tol
+    net.close()
