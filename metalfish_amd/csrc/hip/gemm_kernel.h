@@ -7,10 +7,11 @@
 // row-major, weights in the reference's [out][in] layout).  A workgroup of
 // WM x WN waves owns a BM x BN tile; each wave owns a (BM/WM) x (BN/WN)
 // sub-tile of v_mfma_f32_16x16x32_bf16 instructions.  K advances in BK-wide
-// steps (BK = 32 or 64) through an ST-stage LDS ring filled by
-// global_load_lds_dwordx4 (direct global->LDS, no VGPR round trip): ST - 1
-// steps' tiles are in flight while the current one feeds the MFMAs, enough
-// bytes in flight to cover the L2/HBM latency.  LDS rows
+// steps (BK = 32 or 64) through an ST-stage LDS ring filled by 16-byte loads
+// from global memory straight into LDS (no VGPR round trip): ST - 1 steps'
+// tiles are in flight while the current one feeds the MFMAs, enough bytes in
+// flight to cover the L2/HBM latency.  The pipelined loops also read the next
+// step's fragments, and issue the loads in parts, between the MFMAs.  LDS rows
 // are BK bf16 wide with their 16-byte chunks XOR-swizzled so that the 16 rows
 // a fragment read touches spread over all bank groups; the swizzle is applied
 // on the global side (each lane fetches the chunk that belongs in its LDS
@@ -1722,12 +1723,10 @@ template <int BM, int BN, int BK, int ST, int WM, int WN, bool SPLIT, bool W8, b
           bool PIPE = false, bool LO8 = false>
 hipError_t LaunchW(const GemmParams &p, hipStream_t stream) {
   // A folded LayerNorm (GemmParams::fold_c / out_gamma / res_stats): its
-  // epilogue code is compiled only into the tiles that take it (LnFoldTile:
-  // the pipelined split-precision and BF16X2_FP8LO tiles of the large
-  // batches, the small-LDS split 64 x 64 tile of the smolgen compression
-  // beside Q|K|V and at 24-62 positions where its K is not split, and the
-  // split 64 x 64 tiles of 24-62 positions), bf16 outputs and the residual
-  // mode; the split-K reduce applies it for split consumers.
+  // epilogue code is compiled only into the split-precision tiles that
+  // LargeTile gives such a GEMM (the pipelined ones, the BF16X2_FP8LO one and
+  // the small 64 x 64 one of the compression beside Q|K|V), for bf16 outputs
+  // and the residual mode; the split-K reduce applies it for split consumers.
   constexpr bool kLn = !F8 && (SPLIT || LO8) && (PIPE || (BM == 64 && BN == 64));
   if (p.fold_c || p.out_gamma || p.res_stats) {
     if constexpr (kLn) {

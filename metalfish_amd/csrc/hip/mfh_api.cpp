@@ -1593,7 +1593,11 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
       return rc;
   }
 
-  // Single position (M <= 64 token rows, bf16 weights): the smolgen chain
+  // Dense2's LayerNorm and the global projection in one launch.
+  const bool smolgen_bias =
+      d.smolgen && !d.fused_bias && M < kSmolgenBiasRows && mfh::SmolgenBiasOk(d.H, d.G, kSquares * kSquares);
+  // Single position (M <= 64 token rows, bf16 weights) where the shapes rule
+  // that launch out (over 32 heads, another gen width): the smolgen chain
   // runs as three few-row GEMM launches instead of six (split-K GEMMs with
   // their LayerNorm and reduce launches).  dense1 writes its activated rows
   // with their partial row statistics, dense2 applies dense1's LayerNorm as
@@ -1601,20 +1605,18 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
   // rows one head's gen-wide segment of the position's row).
   const bool few_row_smolgen =
       d.smolgen && d.skinny && M <= mfh::kSkinnyMaxRows && B * d.H <= mfh::kSkinnyMaxRows &&
-      !net->fp8 && !d.fused_bias && d.HG <= 8192 &&
+      !net->fp8 && !d.fused_bias && !smolgen_bias && d.HG <= 8192 &&
       mfh::SkinnyShapeOk(B, d.Hs, kSquares * d.C) && mfh::SkinnyShapeOk(B, d.HG, d.Hs) &&
       mfh::SkinnyShapeOk(B * d.H, kSquares * kSquares, d.G);
   // Up to kSmolgenFewRowMaxBatch positions: dense1 and dense2 (one row per
-  // position) run as few-row GEMMs too, dense2 applying dense1's LayerNorm
-  // as it loads its rows; dense2's LayerNorm and the global projection
-  // (B * H rows) stay separate launches.
+  // position) run as few-row GEMMs, dense2 applying dense1's LayerNorm as it
+  // loads its rows; dense2's LayerNorm and the global projection (B * H rows)
+  // follow.  Also at one position: 1162 -> 1125 us against the three few-row
+  // launches, bf16 1101 -> 1060 (the last of them 9.6 us, now 8).
   const bool few_row_dense = d.smolgen && d.skinny && !few_row_smolgen &&
                              B <= kSmolgenFewRowMaxBatch && !net->fp8 &&
                              mfh::SkinnyShapeOk(B, d.Hs, kSquares * d.C) &&
                              mfh::SkinnyShapeOk(B, d.HG, d.Hs);
-  // Dense2's LayerNorm and the global projection in one launch.
-  const bool smolgen_bias =
-      d.smolgen && !d.fused_bias && M < kSmolgenBiasRows && mfh::SmolgenBiasOk(d.H, d.G, kSquares * kSquares);
   auto run_bias = [&](const mfh::SmolgenBiasParams &p, hipStream_t s) {
     const double rows = static_cast<double>(p.batch) * p.heads;
     const double out_bytes = p.out_lo8 ? 3.0 : p.split ? 4.0 : 2.0;

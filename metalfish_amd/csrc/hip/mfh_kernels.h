@@ -132,14 +132,14 @@ struct GemmParams {
   const float *out_gamma = nullptr;
   float *out_stats = nullptr;
   int ln_width = 0;  // width of the normalised rows (K for ln_stats, N otherwise)
-  // Tiles that leave room for a concurrent launch on another stream (bf16
-  // weights).  beside_chain (split precision): whole-round 256 x 256 tiles
-  // take two LDS stages (96 KiB) instead of three (144 KiB).  small_lds:
-  // below the large-problem rows, 64 x 64 tiles over BK = 32 with two
-  // stages (24 KiB split, 16 KiB single bf16) instead of BK = 64 with three
-  // (72 / 48 KiB), so they fit on a CU beside a two-stage split or a
-  // four-stage single-bf16 256 x 256 tile.  Neither changes the result
-  // bits (the K order of the MFMAs is the same).
+  // Tiles that leave room for a concurrent launch on another stream.
+  // beside_chain: 256 x 256 with two LDS stages (96 KiB) on whole rounds,
+  // else (split) 128 x 256 of four waves with two (64 KiB), so that a CU
+  // takes another workgroup beside.  small_lds: below the large-problem rows,
+  // 64 x 64 tiles over BK = 32 with two stages (24 KiB split, 16 KiB single
+  // bf16; bf16 weights) instead of BK = 64 with three (72 / 48 KiB), for a
+  // launch that runs beside those.  Neither changes the result bits (the K
+  // order of the MFMAs is the same).
   bool beside_chain = false;
   bool small_lds = false;
   // Set by LaunchGemm: every output row start allows 4-column vector stores

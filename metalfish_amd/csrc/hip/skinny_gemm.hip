@@ -19,7 +19,8 @@
 //
 // Measured on MI355X at batch 1 (BT4 shape): the smolgen chain takes 24 us
 // per layer this way against 29.5 us as split-K GEMMs with LayerNorm and
-// reduce launches.  Running every dense layer of the encoder layer this way
+// reduce launches, and 23 with the projection in smolgen_bias.hip, which
+// takes it over where its shapes allow.  Running every dense layer of the encoder layer this way
 // (8 launches per layer instead of 15, residual LayerNorms deferred into the
 // next GEMM) was slower (1.78 vs 1.52 ms per forward): every workgroup reads
 // all 64 activation rows, about 290 KB per CU for the body GEMMs.  Splitting

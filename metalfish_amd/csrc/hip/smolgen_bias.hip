@@ -24,8 +24,8 @@
 // weights) at a few positions, then L2 reads of the weights, which every row
 // group streams whole.  Measured (BT4 shape, split precision) against the
 // LayerNorm and GEMM launches: 8.1 us instead of 5.1 + 4.4 and a launch at
-// batch 8, 18.6 instead of 12.8 + 15.9 at 45; forward 1175 -> 1141 us at batch
-// 2, 1373 -> 1350 at 8, 2489 -> 2443 at 36, 2697 -> 2677 at 45.  From 48
+// batch 8, 18.6 instead of 12.8 + 15.9 at 45; forward 1162 -> 1125 us at batch
+// 1, 1175 -> 1141 at 2, 1373 -> 1350 at 8, 2489 -> 2443 at 36, 2697 -> 2677 at 45.  From 48
 // positions on Q|K|V, on the other stream, outlasts the LayerNorm, and the
 // wider tiles of the GEMM read the weights less often: 48 was 1.2 % slower on
 // this kernel, 64 5 %, 256 4 %, so those keep the two launches.
