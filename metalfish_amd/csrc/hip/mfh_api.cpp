@@ -109,22 +109,20 @@ constexpr int kSmolgenBiasRows = 48 * kSquares;
 // BF16X2_FP8LO: the fp8 lo correction runs from this many token rows (128
 // positions); below, the forward is the BF16X2 one.
 constexpr int kLo8MinRows = 8192;
-// From this many token rows (24 positions) the body's residual LayerNorms
-// are folded into the GEMMs around them (GemmParams: the residual GEMMs write
-// x o gamma with per-row partial sums, Q|K|V, the compression and FFN1 take
-// the LayerNorm in their epilogue, the next residual rebuilds it).
+// The body's residual LayerNorms are folded into the GEMMs around them
+// (GemmParams: the residual GEMMs write x o gamma with per-row partial sums,
+// Q|K|V, the compression and FFN1 take the LayerNorm in their epilogue, the
+// next residual rebuilds it) from kFoldRows token rows (24 positions) while
+// the residual GEMMs (N = E) have fewer 128 x 128 tiles than CUs (up to 62
+// positions at E = 1024), and, in nets sized for kFoldWholeRows (256
+// positions), where those GEMMs take whole rounds of 256 x 256 tiles.
+// Elsewhere the LayerNorm kernels run although the fold is the faster there
+// too (one box: batch 100 5287 -> 4999 us, 200 8699 -> 8234, 300 13181 ->
+// 12463): it stores x o gamma where they store LN(x), so rounding counts
+// relative to |x| instead of |x - mean|, and calls that did not have that
+// trade do not get it.
 constexpr long kFoldRows = 1536;
-// (Fold measured against the LayerNorm kernels, one box: batch 48 3042 ->
-// 2777 us, 100 5287 -> 4999, 200 8699 -> 8234, 300 13181 -> 12463, 600 25877
-// -> 24432, 1000 41469 -> 39378.)  Very large residual streams whose N = E
-// GEMMs stop just short of whole rounds of 256 x 256 tiles keep the
-// kernels, as they always did (from kFoldShortElements elements and the
-// last round 9 / 10 full on).
-constexpr long kFoldShortElements = 32000000;
-bool StopsShortOfWholeRounds(long rows, long width) {
-  const long last = (rows + 255) / 256 * ((width + 255) / 256) % 256;
-  return rows * width >= kFoldShortElements && 10 * last >= 9 * 256;
-}
+constexpr long kFoldWholeRows = 16384;
 
 std::uint16_t ToBf16(float f) {
   std::uint32_t u;
@@ -280,8 +278,8 @@ struct mfh_net {
   // offset of its e4m3 codes.
   std::map<size_t, size_t> lo8_codes;
   // The body's fold constants were packed (Layer::qkv_fold / ffn1_fold),
-  // for kFoldRows token rows.
-  bool has_fold = false;
+  // for kFoldRows token rows; also for kFoldWholeRows.
+  bool has_fold = false, has_fold_whole = false;
   size_t head_b, qk_b, promo, val1_b, val2_w, val2_b, gather;
   size_t head_w[2], qk_w[2], val1_w[2];
   size_t mov_b = 0, mov1_b = 0, mov2_w = 0, mov2_b = 0;  // moves-left head
@@ -920,6 +918,7 @@ int Pack(mfh_net *net, Loader &ld, Blob &blob) {
                 L.ffn1_fold);
     }
     net->has_fold = true;
+    net->has_fold_whole = net_rows >= kFoldWholeRows;
   }
   // Policy encoder layers (weights.cpp:188-203), no smolgen.
   net->pol_layers.resize(d.PL);
@@ -1323,8 +1322,12 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
   // kFoldRows): the whole forward (a single debug layer keeps them).
   // (Checked below: every GEMM around them must have a tile that compiles
   // the folded epilogue.)
+  const auto tiles128 = [&](int n) {
+    return static_cast<long>((M + 127) / 128) * ((n + 127) / 128);
+  };
+  const bool fold_whole = net->has_fold_whole && whole_round(M, E);
   bool fold = net->has_fold && full && ws.Has("st_act") && M >= kFoldRows &&
-              !StopsShortOfWholeRounds(M, E);
+              (fold_whole || tiles128(E) < 256);
   float *st_act = nullptr, *st_mid = nullptr;
   auto ln = [&](const float *x, int rows, int width, float eps, const float *g, const float *b,
                 float *y32, const std::string &y16) {
@@ -1738,8 +1741,15 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
     mfh::GemmParams p2 = gemm("hid", d.F, L.ffn2_w, d.F, M, E, d.F, nullptr, mfh::ACT_NONE, res,
                               nullptr, nullptr, E);
     use_lo8(p2, "hid", L.ffn2_w);
-    fold = (li == 0 || mfh::GemmLnFoldOk(pq)) && (li == 0 || !L.smolgen || mfh::GemmLnFoldOk(pc)) &&
-           mfh::GemmLnFoldOk(pf) && mfh::GemmLnFoldOk(po) && mfh::GemmLnFoldOk(p2);
+    // (FFN1 on part of a 128-wide tile only at few rows, and below whole
+    // rounds no BF16X2_FP8LO tiles.)
+    if (d.F % 128 && tiles128(d.F) >= (d.F <= 2048 ? 512 : 256))
+      fold = false;
+    if (!fold_whole && (pq.A_lo8 || pf.A_lo8 || po.A_lo8 || p2.A_lo8))
+      fold = false;
+    fold = fold && (li == 0 || mfh::GemmLnFoldOk(pq)) &&
+           (li == 0 || !L.smolgen || mfh::GemmLnFoldOk(pc)) && mfh::GemmLnFoldOk(pf) &&
+           mfh::GemmLnFoldOk(po) && mfh::GemmLnFoldOk(p2);
   }
   if (fold) {
     st_act = ws.S<float>("st_act");
