@@ -178,15 +178,10 @@ __global__ __launch_bounds__(kNarrowWaves * 64, 2) void NarrowKernel(GemmParams 
 #endif
 }
 
-template <bool SPLIT, bool W8>
+template <bool SPLIT, bool W8, bool LN>
 hipError_t LaunchNarrowW(const GemmParams &p, hipStream_t stream) {
   const dim3 grid((p.M + kNarrowTile - 1) / kNarrowTile, (p.N + kNarrowTile - 1) / kNarrowTile);
-  if (p.fold_c)
-    hipLaunchKernelGGL((NarrowKernel<SPLIT, W8, true>), grid, dim3(kNarrowWaves * 64), 0, stream,
-                       p);
-  else
-    hipLaunchKernelGGL((NarrowKernel<SPLIT, W8, false>), grid, dim3(kNarrowWaves * 64), 0, stream,
-                       p);
+  hipLaunchKernelGGL((NarrowKernel<SPLIT, W8, LN>), grid, dim3(kNarrowWaves * 64), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -197,15 +192,20 @@ hipError_t LaunchNarrowW(const GemmParams &p, hipStream_t stream) {
 // slower, 128 2.4 %, 300 2 %.
 constexpr int kNarrowRows = 1088, kNarrowRowsEnd = 3072;
 bool NarrowOk(const GemmParams &p) {
-  return p.M >= kNarrowRows && p.M < kNarrowRowsEnd && p.N < 128 && p.N % 4 == 0 && p.K % (32 * kNarrowWaves) == 0 &&
-         p.k_splits == 1 && p.out_mode == GEMM_OUT_BF16 && p.act == ACT_NONE && !p.A8 &&
-         !p.A_lo8 && !p.C_lo8 && p.split_n >= p.N;
+  return p.M >= kNarrowRows && p.M < kNarrowRowsEnd && p.N < 128 && p.N % 4 == 0 &&
+         p.K % (32 * kNarrowWaves) == 0 && p.k_splits == 1 && p.out_mode == GEMM_OUT_BF16 &&
+         p.act == ACT_NONE && !p.A8 && !p.A_lo8 && !p.C_lo8 && p.split_n >= p.N &&
+         (!p.fold_c || (p.A_lo && !p.W8));
 }
 
 hipError_t LaunchNarrow(const GemmParams &p, hipStream_t stream) {
+  if (p.fold_c)
+    return LaunchNarrowW<true, false, true>(p, stream);
   if (p.A_lo)
-    return p.W8 ? LaunchNarrowW<true, true>(p, stream) : LaunchNarrowW<true, false>(p, stream);
-  return p.W8 ? LaunchNarrowW<false, true>(p, stream) : LaunchNarrowW<false, false>(p, stream);
+    return p.W8 ? LaunchNarrowW<true, true, false>(p, stream)
+                : LaunchNarrowW<true, false, false>(p, stream);
+  return p.W8 ? LaunchNarrowW<false, true, false>(p, stream)
+              : LaunchNarrowW<false, false, false>(p, stream);
 }
 
 // A tile with bf16 or fp8 weights on the pipelined loops.
@@ -386,7 +386,7 @@ int RowsFirst(const GemmParams &p) {
 Tile LargeTile(const GemmParams &p) {
   const bool res = p.out_mode == GEMM_OUT_RESID_F32;
   const bool ln = p.fold_c || p.out_gamma || p.res_stats;
-  if (p.A8 || p.k_splits != 1 || p.K % 64)
+  if (p.A8 || p.k_splits != 1 || p.K % 64 || (ln && p.W8))
     return Tile::kNone;
   if (p.A_lo8)
     return !ln || p.N % 256 == 0 ? Tile::kLo8 : Tile::kNone;

@@ -1723,11 +1723,12 @@ template <int BM, int BN, int BK, int ST, int WM, int WN, bool SPLIT, bool W8, b
           bool PIPE = false, bool LO8 = false>
 hipError_t LaunchW(const GemmParams &p, hipStream_t stream) {
   // A folded LayerNorm (GemmParams::fold_c / out_gamma / res_stats): its
-  // epilogue code is compiled only into the split-precision tiles that
-  // LargeTile gives such a GEMM (the pipelined ones, the BF16X2_FP8LO one and
-  // the small 64 x 64 one of the compression beside Q|K|V), for bf16 outputs
-  // and the residual mode; the split-K reduce applies it for split consumers.
-  constexpr bool kLn = !F8 && (SPLIT || LO8) && (PIPE || (BM == 64 && BN == 64));
+  // epilogue code is compiled only into the split-precision tiles with bf16
+  // weights that LargeTile gives such a GEMM (the pipelined ones, the
+  // BF16X2_FP8LO one and the small 64 x 64 one of the compression beside
+  // Q|K|V), for bf16 outputs and the residual mode; the split-K reduce
+  // applies it for split consumers.
+  constexpr bool kLn = !W8 && !F8 && (SPLIT || LO8) && (PIPE || (BM == 64 && BN == 64));
   if (p.fold_c || p.out_gamma || p.res_stats) {
     if constexpr (kLn) {
       if constexpr (BN >= kLnStatCols)

@@ -532,10 +532,11 @@ int Infer(const mfh_net_desc &desc, Loader &ld, Dims &d) {
   d.split = desc.precision == MFH_PRECISION_BF16X2 ||
             desc.precision == MFH_PRECISION_BF16X2_GEMM || d.lo8;
   d.split_attn = desc.precision == MFH_PRECISION_BF16X2 || d.lo8;
-  // The panel only when asked for: since the e4m3 rows too run on the
-  // pipelined tiles with the LayerNorms folded, batch 1024 takes 38.6 ms
-  // against 44.6 with the panel (BF16X2; the panel had won over the
-  // lock-step e4m3 tiles).  The panel has no fp8 lo correction.
+  // The panel only when asked for: the tiled GEMMs with the LayerNorm kernel
+  // are faster, with e4m3 weights too since those run on the pipelined tiles
+  // (BF16X2, panel -> tiles: batch 128 7499 -> 5762 us, 256 10494 -> 10139,
+  // 300 15157 -> 12493, 1024 41777 -> 40427).  The panel has no fp8 lo
+  // correction.
   d.fused_ln = !d.lo8 && desc.fused_layernorm != 0;
   d.wdl = desc.value == MFH_VALUE_WDL;
   d.mlh = desc.moves_left == 1;
@@ -657,9 +658,12 @@ int Infer(const mfh_net_desc &desc, Loader &ld, Dims &d) {
   // kFoldRows (on unless METALFISH_HIP_FOLD_LN=0).  The folded GEMMs work on
   // x o gamma and subtract mu (W . gamma) after the product, so the rounding
   // of the stored rows counts relative to |x| rather than to |x - mu|: a
-  // row whose mean is large against its spread loses that factor.
+  // row whose mean is large against its spread loses that factor.  Encoder
+  // GEMMs on e4m3 weights have no such epilogue: they keep LN(x) (BF16X2_FP8LO
+  // holds e4m3 weights as scaled bf16 rows, which fold).
   const char *fold_env = std::getenv("METALFISH_HIP_FOLD_LN");
-  d.fold_ln = !(fold_env && fold_env[0] == '0');
+  d.fold_ln = !(fold_env && fold_env[0] == '0') &&
+              (d.lo8 || desc.weights_dtype == MFH_WEIGHTS_BF16);
   // BF16X2_FP8LO: the lo pass of the encoder GEMMs takes 128-byte K steps
   // over code rows laid out 128-byte aligned (K = the embedding and FFN
   // widths, in the body, the input-embedding FFN and policy encoder layers).

@@ -51,3 +51,29 @@ def test_fold_range(precision, monkeypatch):
         if not fewer:
             assert np.array_equal(got["policy"], want["policy"]), b
             assert np.array_equal(got["wdl"], want["wdl"]), b
+
+
+@pytest.mark.parametrize("precision", ["bf16x2", "bf16x2_gemm"])
+def test_e4m3_weights_do_not_fold(precision, monkeypatch):
+    """Nets on e4m3 weights keep the LayerNorm kernels at every batch: the
+    bits and launches of METALFISH_HIP_FOLD_LN=0."""
+    spec = dataclasses.replace(synth.SPECS["bt4"], name="two", layers=2)
+    weights = _off_centre(spec, 5)
+    planes, _ = synth.playout_positions(4, seed=7)
+    outs = {}
+    for env in ("1", "0"):
+        monkeypatch.setenv("METALFISH_HIP_FOLD_LN", env)
+        net = backend.create_network(spec, weights, max_batch=256, device=0, precision=precision,
+                                     weights_dtype="fp8")
+        assert "e4m3" in net.info()
+        net.set_profiling(True)
+        for b in (24, 47, 62, 100, 256):
+            net.profile_reset()
+            out = net.evaluate_batch(planes[np.arange(b) % 4])
+            outs[env, b] = out, net.profile()["layernorm"]["launches"]
+        net.close()
+    for (env, b), (got, launches) in outs.items():
+        want, kernels = outs["0", b]
+        assert launches == kernels, b
+        assert np.array_equal(got["policy"], want["policy"]), b
+        assert np.array_equal(got["wdl"], want["wdl"]), b
