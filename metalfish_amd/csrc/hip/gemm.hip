@@ -3,6 +3,8 @@
 #include "gemm_kernel.h"
 #include "gemm_tiles.h"
 
+#include <algorithm>
+
 namespace mfh {
 MFH_TILES(MFH_TILE_DECLARE)
 
@@ -446,11 +448,29 @@ GemmParams RowRange(const GemmParams &p, int first, int rows) {
   q.resid16 = bf16(p.resid16, r * p.ldr);
   q.resid16_lo = bf16(p.resid16_lo, r * p.ldr);
   q.C_lo8 = p.C_lo8 ? p.C_lo8 + r * p.ldc8 : nullptr;
+  q.A_lo8 = p.A_lo8 ? p.A_lo8 + r * p.lda8 : nullptr;
   const size_t stats = p.ln_width ? r * (p.ln_width / kLnStatCols) * 2 : 0;
   q.ln_stats = p.ln_stats ? p.ln_stats + stats : nullptr;
   q.res_stats = p.res_stats ? p.res_stats + stats : nullptr;
   q.out_stats = p.out_stats ? p.out_stats + stats : nullptr;
   return q;
+}
+
+// The pipelined tiles address an operand with 32-bit byte offsets from its
+// first element, below 2^31 (past that a buffer load reads zeros).  Rows of p
+// within reach: all of them, or how many to take at a time, in equal ranges of
+// whole 256-row tiles (0: the weights, or 256 rows, are past it).
+constexpr long kReach = (1l << 31) - 1;
+int RowsInReach(const GemmParams &p) {
+  if (static_cast<long>(p.N) * p.ldw * (p.W8 ? 1 : 2) > kReach)
+    return 0;
+  const long most = kReach / (2l * p.lda);
+  if (p.M <= most)
+    return p.M;
+  if (most < 256 || p.k_splits > 1)  // (a slice's plane holds all rows)
+    return 0;
+  const long ranges = (p.M + most / 256 * 256 - 1) / (most / 256 * 256);
+  return static_cast<int>(((p.M + ranges - 1) / ranges + 255) / 256 * 256);
 }
 
 hipError_t LaunchTile(Tile t, const GemmParams &p, hipStream_t stream) {
@@ -658,11 +678,27 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
            (p.out_mode != GEMM_OUT_RESID_F32 ||
             (p.resid16 ? Aligned(p.resid16, 16) && Aligned(p.resid16_lo, 16) && p.ldr % 8 == 0
                        : Aligned(p.resid, 16) && p.ldr % 4 == 0));
-  // Large shapes and any folded LayerNorm: the tiles of LargeTile.  (BF16X2_FP8LO: 256 x 256 tiles of
-  // eight waves, the hi pass on the four-stage single-bf16 pipelined ring,
-  // 128 KiB, then the lo pass on two 64 KiB stages of code rows.)
   if (NarrowOk(p))
     return LaunchNarrow(p, stream);
+  const int reach = f8 ? p.M : RowsInReach(p);
+  if (reach == 0) {
+    // Lock-step tiles, which load through 64-bit addresses.
+    if (p.fold_c || ln_res || lo8)
+      return fail("folded LayerNorm or fp8 lo correction: weights below 2 GiB");
+    return p.A_lo ? LaunchStep32<true>(p, stream) : LaunchStep32<false>(p, stream);
+  }
+  if (reach < p.M) {
+    for (int first = 0; first < p.M; first += reach) {
+      const GemmParams q = RowRange(p_in, first, std::min(reach, p.M - first));
+      const hipError_t e = LaunchGemm(q, stream, err);
+      if (e != hipSuccess)
+        return e;
+    }
+    return hipSuccess;
+  }
+  // Large shapes and any folded LayerNorm: the tiles of LargeTile.  (BF16X2_FP8LO: 256 x 256 tiles
+  // of eight waves, the hi pass on the four-stage single-bf16 pipelined ring,
+  // 128 KiB, then the lo pass on two 64 KiB stages of code rows.)
   const Tile tile = LargeTile(p);
   if (tile == Tile::kSplitK) {
     if (!Aligned(p.partials, 16) || !p.vec || p.N % 4)

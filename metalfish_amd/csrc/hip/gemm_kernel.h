@@ -451,8 +451,8 @@ constexpr int GemmStageBytes() {
 // (The buffer-resource type exists only in the device pass.)
 #if defined(__HIP_DEVICE_COMPILE__)
 // Buffer resource over a whole operand (raw addressing: stride 0, byte
-// offsets below 2^31; the loads' offsets are clamped to valid rows, so the
-// range check never triggers).
+// offsets below 2^31, which LaunchGemm sees to; the loads' offsets are clamped
+// to valid rows, so the range check never triggers).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t BufferRsrc(const void *base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0x7FFFFFFF, 0x00020000);
 }

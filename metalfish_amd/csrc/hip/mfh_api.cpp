@@ -1509,7 +1509,8 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
                          const float *g, const float *b, float *y32, bool f8 = false) -> int {
     // fused_layernorm: the panel streams each weight row from L2 for only 64
     // activation rows.
-    if (d.fused_ln && d.split && M >= kPanelMinRows &&
+    // (Its 32-bit offsets reach operands below 2 GiB.)
+    if (d.fused_ln && d.split && M >= kPanelMinRows && 2.0 * M * k < 2147483648.0 &&
         mfh::PanelGemmShapeOk(mfh::PANEL_OUT_LN, E, k)) {
       mfh::PanelGemmParams pp;
       pp.A = ws.S<std::uint16_t>(a);

@@ -52,6 +52,50 @@ def test_large_tiles_equal_small_ones(m, n, k, act):
         assert (np.abs(small - z) <= bound).all()
 
 
+@pytest.mark.parametrize("m,n,k", [(2_200_000, 64, 1024), (1_060_000, 128, 1024),
+                                   (64, 2_200_000, 1024), (1536, 700_032, 1600),
+                                   (300, 66, 1 << 22)])
+def test_operands_past_2_and_4_gib(m, n, k):
+    """Operands of more than 2 and 4 GiB, which the pipelined tiles' 32-bit
+    offsets do not reach (activations: taken in ranges of rows; weights, or
+    rows too long for a range: lock-step tiles): rows on both sides of the
+    limits equal those of a small call, to the bit.  (Zeros elsewhere, which
+    a wrapped or range-checked address would read.)"""
+    rng = np.random.default_rng(m + n)
+
+    def picked(count):
+        if count <= 70:
+            return list(range(count))
+        near = [limit // (2 * k) + i for limit in (1 << 31, 1 << 32) for i in (-1, 0, 1)]
+        return sorted({i for i in near + [0, 1, count // 2, count - 66, count - 1] if i < count})
+
+    rows, cols = picked(m), picked(n)
+    a, w = np.zeros((m, k), np.uint16), np.zeros((n, k), np.uint16)
+    at = slice(k - 1024, k)
+    a[rows, at] = _bits(rng, (len(rows), 1024))
+    w[cols, at] = _bits(rng, (len(cols), 1024), 1 / 32)
+    out = backend.gemm_bf16(a, w)
+    small = backend.gemm_bf16(a[rows][:, at], w[cols][:, at])
+    assert np.count_nonzero(small) == small.size
+    assert np.array_equal(out[np.ix_(rows, cols)].view(np.uint32), small.view(np.uint32))
+
+
+def test_lo8_rows_past_2_gib():
+    """The same for activations with e4m3 lo codes, bf16 output and codes."""
+    m, n, k = 1_100_000, 64, 1024
+    rng = np.random.default_rng(3)
+    rows = [0, 1, m // 2, (1 << 20) - 1, 1 << 20, (1 << 20) + 1, m - 66, m - 1]
+    a, a8 = np.zeros((m, k), np.uint16), np.zeros((m, k), np.uint8)
+    a[rows] = _bits(rng, (len(rows), k))
+    a8[rows] = rng.integers(0, 0x40, (len(rows), k))
+    w, w8 = _bits(rng, (n, k), 1 / 32), rng.integers(0, 0x40, (n, k)).astype(np.uint8)
+    scale = np.full(n, 0.5, np.float32)
+    out = backend.gemm_lo8(a, a8, w, w8, scale, bf16_out=True)
+    small = backend.gemm_lo8(a[rows], a8[rows], w, w8, scale, bf16_out=True)
+    for got, want in zip(out, small):
+        assert np.array_equal(got[rows], want)
+
+
 @pytest.mark.parametrize("weights_dtype", ["bf16", "fp8"])
 @pytest.mark.parametrize("precision", ["bf16x2", "bf16x2_gemm", "bf16"])
 def test_batches_across_tile_rules_agree(precision, weights_dtype):
