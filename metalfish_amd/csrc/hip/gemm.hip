@@ -367,7 +367,7 @@ bool StoreBound(const GemmParams &p) {
 // nearly empty costs as much as a full one: out-projection at 19200 rows
 // (300 tiles of 256 x 256) 129 us on them, 100 on 128 x 128, 67 + 20 split.
 int RowsFirst(const GemmParams &p) {
-  if (p.N % 256 || p.beside_chain || p.M < kLargeRows || StoreBound(p))
+  if (p.N % 256 || p.K % 64 || p.beside_chain || p.M < kLargeRows || StoreBound(p))
     return 0;
   const TileTime &whole = p.A_lo ? kTileTimes[0] : kOneTimes[0];
   const int nbn = p.N / 256, nbm = p.M / 256;
@@ -388,8 +388,16 @@ int RowsFirst(const GemmParams &p) {
 Tile LargeTile(const GemmParams &p) {
   const bool res = p.out_mode == GEMM_OUT_RESID_F32;
   const bool ln = p.fold_c || p.out_gamma || p.res_stats;
-  if (p.A8 || p.k_splits != 1 || p.K % 64 || (ln && p.W8))
+  if (p.A8 || p.k_splits != 1 || (ln && p.W8))
     return Tile::kNone;
+  if (p.K % 64) {
+    // The tiles over BK = 32, on whole rounds.  Isolated, single bf16, against
+    // the lock-step 64 x 64 ones: 16384 x 1024 over K = 1056 104 -> 52 us,
+    // 65536 x 256 over 224 42 -> 27, 16384 x 1024 over 96 28 -> 24.
+    if (ln || p.A_lo8 || !GemmWholeRoundTiles(p))
+      return Tile::kNone;
+    return !p.A_lo ? Tile::kOne256 : p.beside_chain ? Tile::k256Two : Tile::k256;
+  }
   if (p.A_lo8)
     return !ln || p.N % 256 == 0 ? Tile::kLo8 : Tile::kNone;
   if (!p.A_lo) {

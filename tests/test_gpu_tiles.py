@@ -25,7 +25,7 @@ def _bits(rng, shape, scale=1.0):
                                    (2047, 1024, 1024), (4096, 1024, 1024), (4100, 1536, 1024),
                                    (6400, 1024, 1536), (12800, 256, 192), (16385, 256, 64),
                                    (16640, 1024, 256), (1536, 1056, 96), (2048, 2048, 256),
-                                   (1601, 2304, 128), (256, 1536, 1024), (511, 3136, 1024),
+                                   (1601, 2304, 128), (16384, 1024, 224), (256, 1536, 1024), (511, 3136, 1024),
                                    (700, 1538, 512), (1030, 3136, 1024), (1535, 1536, 640)])
 @pytest.mark.parametrize("act", ["none", "mish"])
 def test_large_tiles_equal_small_ones(m, n, k, act):
