@@ -122,8 +122,9 @@ typedef struct {
   int fused_layernorm;    /* residual GEMM + the LayerNorm after it as one
                              row-panel launch (batches >= 128, BF16X2 and
                              BF16X2_GEMM): 1 always; 0 chooses as measured on
-                             MI355X: off (tiled GEMMs with the LayerNorm kernel,
-                             or the LayerNorm folded into them) */
+                             MI355X: on with fp8 weights of width 256, else off
+                             (tiled GEMMs with the LayerNorm kernel, or the
+                             LayerNorm folded into them) */
 } mfh_net_desc;
 
 /* One weight tensor, named as in the reference's weight inventory

@@ -532,12 +532,6 @@ int Infer(const mfh_net_desc &desc, Loader &ld, Dims &d) {
   d.split = desc.precision == MFH_PRECISION_BF16X2 ||
             desc.precision == MFH_PRECISION_BF16X2_GEMM || d.lo8;
   d.split_attn = desc.precision == MFH_PRECISION_BF16X2 || d.lo8;
-  // The panel only when asked for: the tiled GEMMs with the LayerNorm kernel
-  // are faster, with e4m3 weights too since those run on the pipelined tiles
-  // (BF16X2, panel -> tiles: batch 128 7499 -> 5762 us, 256 10494 -> 10139,
-  // 300 15157 -> 12493, 1024 41777 -> 40427).  The panel has no fp8 lo
-  // correction.
-  d.fused_ln = !d.lo8 && desc.fused_layernorm != 0;
   d.wdl = desc.value == MFH_VALUE_WDL;
   d.mlh = desc.moves_left == 1;
   d.act_default = desc.default_activation == MFH_DEFAULT_ACTIVATION_MISH ? mfh::ACT_MISH
@@ -548,6 +542,15 @@ int Infer(const mfh_net_desc &desc, Loader &ld, Dims &d) {
   // Shapes follow from bias sizes, as in the reference's shape inference
   // (network_execution_plan.cpp:279-289).
   d.E = static_cast<int>(ld.Count("body.ip_emb_b"));
+  // The panel when asked for, and by itself with e4m3 weights of width 256
+  // (BF16X2, FFN 512, tiles and LayerNorm kernel -> panel: 160 positions 637
+  // -> 618 us, 256 816 -> 717, 512 1259 -> 1183, 1024 2302 -> 2170; FFN 1024
+  // 128 604 -> 622, 256 903 -> 805, 1024 2599 -> 2680).  Wider nets take the
+  // tiles: 512 within 9 % either way, 768 at 128 1258 -> 1476, 1024 at 128
+  // 5762 -> 7499, 256 10139 -> 10494, 300 12493 -> 15157, 1024 40427 ->
+  // 41777.  The panel has no fp8 lo correction.
+  d.fused_ln = !d.lo8 && (desc.fused_layernorm != 0 ||
+                          (desc.weights_dtype == MFH_WEIGHTS_FP8 && d.E == 256));
   d.pe_map = desc.input_embedding == MFH_INPUT_EMBEDDING_PE_MAP;
   // PE_MAP: the static encoding's width is what the embedding dense takes
   // beyond the 112 planes (network_execution_plan.cpp:833-865).

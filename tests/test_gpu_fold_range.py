@@ -77,3 +77,30 @@ def test_e4m3_weights_do_not_fold(precision, monkeypatch):
         assert launches == kernels, b
         assert np.array_equal(got["policy"], want["policy"]), b
         assert np.array_equal(got["wdl"], want["wdl"]), b
+
+
+def test_e4m3_weights_of_width_256_take_the_row_panel():
+    """From 128 positions (8192 rows) nets of width 256 on e4m3 weights run
+    their residual GEMMs with the LayerNorm in one row-panel launch without
+    being asked to (2L + 1 = 5 LayerNorm launches fewer than at 127), wider
+    ones do not."""
+    planes, _ = synth.playout_positions(4, seed=7)
+    wide = dataclasses.replace(synth.SPECS["cpu_plumbing"], name="wide", embedding=512, heads=16)
+    for spec, fewer in ((synth.SPECS["cpu_plumbing"], 5), (wide, 0)):
+        weights = synth.make_weights(spec, seed=1, fp8=True)
+        outs = []
+        for fused in (False, True):
+            net = backend.create_network(spec, weights, max_batch=128, device=0,
+                                         weights_dtype="fp8", fused_layernorm=fused)
+            net.set_profiling(True)
+            launches = []
+            for b in (127, 128):
+                net.profile_reset()
+                out = net.evaluate_batch(planes[np.arange(b) % 4])
+                launches.append(net.profile()["layernorm"]["launches"])
+            net.close()
+            outs.append(out)
+            assert launches[1] == launches[0] - (5 if fused else fewer), (spec.name, launches)
+        if fewer:
+            assert np.array_equal(outs[0]["policy"], outs[1]["policy"])
+        assert np.abs(outs[0]["policy"] - outs[1]["policy"]).max() <= 1e-4
