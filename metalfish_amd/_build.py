@@ -28,9 +28,10 @@ HIP_SOURCES = ["hip/gemm_tiles_pipe_a.hip", "hip/gemm_tiles_pipe_b.hip",
                "hip/gemm_tiles_pipe_c.hip", "hip/gemm_tiles_single_mid.hip",
                "hip/gemm_tiles_single.hip", "hip/gemm_tiles_mid.hip", "hip/gemm_tiles_small.hip",
                "hip/gemm_tiles_w8_a.hip", "hip/gemm_tiles_w8_b.hip", "hip/gemm_tiles_w8_c.hip",
-               "hip/gemm_tiles_w8_single.hip", "hip/gemm_tiles_w8_small.hip", "hip/gemm.hip", "hip/panel_gemm.hip", "hip/skinny_gemm.hip", "hip/smolgen_bias.hip", "hip/attention.hip", "hip/rowops.hip",
-               "hip/policy.hip",
-               "hip/mfh_api.cpp", "host/policy_tables.cpp"]
+               "hip/gemm_tiles_w8_single.hip", "hip/gemm_tiles_w8_small.hip", "hip/gemm.hip",
+               "hip/panel_gemm.hip", "hip/skinny_gemm.hip", "hip/smolgen_bias.hip",
+               "hip/attention.hip", "hip/rowops.hip", "hip/policy.hip", "hip/mfh_api.cpp",
+               "host/policy_tables.cpp"]
 # Host-only parts of libmfhip.so (no device code), compiled with g++.
 HIP_HOST_SOURCES = ["host/weights_file.cpp", "host/pack_planes.cpp"]
 HOST_SOURCES = ["host/chess.cpp", "host/policy_tables.cpp", "host/synth_api.cpp"]

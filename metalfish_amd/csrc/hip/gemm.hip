@@ -358,8 +358,8 @@ Tile BestTile(const GemmParams &p, int M, float *us) {
 // 9600 35.7 (256 x 128 39.7), 16384 56.3 (60.7), 32768 131 (122.9).  Past 16384
 // rows the 256 x 256 tiles' rounds are long enough (batch 1024 0.6 % slower).
 bool StoreBound(const GemmParams &p) {
-  return p.K <= 256 && p.M > 2048 && p.M <= 16384 && p.N >= 2048 && p.N % 256 == 0 && p.act == ACT_NONE && !p.beside_chain &&
-         p.out_mode != GEMM_OUT_RESID_F32 && !p.fold_c;
+  return p.K <= 256 && p.M > 2048 && p.M <= 16384 && p.N >= 2048 && p.N % 256 == 0 &&
+         p.act == ACT_NONE && !p.beside_chain && p.out_mode != GEMM_OUT_RESID_F32 && !p.fold_c;
 }
 
 // Rows of p to run on whole rounds of 256 x 256 tiles, the rest following as
@@ -716,7 +716,8 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
     if (rows == 0)
       return LaunchTile(tile, p, stream);
     float us;
-    const hipError_t e = LaunchTile(p.A_lo ? Tile::k256 : Tile::kOne256, RowRange(p, 0, rows), stream);
+    const Tile whole = p.A_lo ? Tile::k256 : Tile::kOne256;
+    const hipError_t e = LaunchTile(whole, RowRange(p, 0, rows), stream);
     const GemmParams rest = RowRange(p, rows, p.M - rows);
     return e != hipSuccess ? e : LaunchTile(BestTile(rest, rest.M, &us), rest, stream);
   } else if (p.fold_c || ln_res || lo8) {
@@ -773,8 +774,8 @@ hipError_t LaunchGemm(const GemmParams &p_in, hipStream_t stream, std::string *e
   // (21.8); FFN1 at 768 11.1 on 64 x 128 (12.4); single bf16 Q|K|V at 1024 12.4
   // on 128 x 128 (16.5).  (Beside the chain, from 17 positions, the 128 x 128
   // tiles' 144 KiB keep its workgroups off the CU: batch 20 4 % slower.)
-  if (p.M >= kModelRows && p.M < (p.W8 ? kLargeRows : kModelRowsEnd) && p.N >= 128 && p.k_splits == 1 && p.K % 64 == 0 &&
-      p.K >= 512 && !p.small_lds && !p.beside_chain) {
+  if (p.M >= kModelRows && p.M < (p.W8 ? kLargeRows : kModelRowsEnd) && p.N >= 128 &&
+      p.k_splits == 1 && p.K % 64 == 0 && p.K >= 512 && !p.small_lds && !p.beside_chain) {
     float us;
     return LaunchTile(BestTile(p, p.M, &us), p, stream);
   }

@@ -383,10 +383,6 @@ __device__ __forceinline__ void Epilogue8(const GemmParams &p, int row, int col,
   Finish8<MODE, ACT>(p, row, col, v, b, rv);
 }
 
-// The folded-LayerNorm residual epilogue: a thread keeps one column group
-// for the tile (the threads are a multiple of the groups per row and every
-// thread runs the same rows) and each 128-column block of a row is 16
-// consecutive lanes (tiles 128 or 256 columns wide).
 // Rows per pass of the staged epilogue: the fp32 tile rows (BN + 4 floats
 // each) that fit the LDS ring of ST stages of STAGE_BYTES.
 template <int BM, int BN, int ST, int STAGE_BYTES>
@@ -399,9 +395,13 @@ constexpr int StagedRows() {
          : ring >= 32 * pitch  ? 32
                                : 16;
 }
+// The folded-LayerNorm residual epilogue: a thread keeps one column group
+// for the tile (the threads are a multiple of the groups per row and every
+// thread runs the same rows) and each 128-column block of a row is 16
+// consecutive lanes (tiles 128 or 256 columns wide).
 template <int BN, int THREADS, int RB>
 constexpr bool GemmLnEpilogueOk() {
-  return (BN == 64 || BN == 128 || BN == 256) && THREADS % (BN / 8) == 0 &&
+  return (BN == 128 || BN == 256) && THREADS % (BN / 8) == 0 &&
          (RB * (BN / 8)) % THREADS == 0;
 }
 
@@ -422,7 +422,7 @@ constexpr int GemmStageBytes() {
   return !W8 ? a + BN * BK * 2 : W8InLds<BM, BN, BK, WM, WN, SPLIT>() ? a + BN * BK : a;
 }
 
-// Software-pipelined main loop (bf16 weights, BK = 32): LDS fragment reads
+// Software-pipelined main loop (BK = 32): LDS fragment reads
 // for the next MFMAs are issued while earlier MFMAs run, so neither the LDS
 // latency nor the LDS pipe's time opens a gap in the MFMA stream.  In the
 // lock-step loop the compiler waited for each group of fragment reads just
@@ -757,9 +757,8 @@ __device__ __forceinline__ void PipelinedLoop(const GemmParams &p, std::uint16_t
   }
 }
 
-// Software-pipelined main loop over BK = 64 stages (bf16 weights), for tiles
-// too small to hide a barrier and an LDS latency behind one 32-wide K step's
-// MFMAs.  A stage is two 32-wide substeps and has one barrier; the fragments
+// Software-pipelined main loop over BK = 64 stages, for tiles too small to
+// hide a barrier and an LDS latency behind one 32-wide K step's MFMAs.  A stage is two 32-wide substeps and has one barrier; the fragments
 // are double-buffered in registers: a substep's MFMAs run on one set while
 // the other set is read for the next substep, a whole substep ahead of its
 // use.  A 32-wide step of a 128 x 128 split tile takes 0.28 us this way
@@ -1118,7 +1117,7 @@ __global__ __launch_bounds__(WM *WN * 64, PIPE && WM * WN == 4 ? 2 : 1) void Gem
   // Each lane's source pointer for its LPW wave-loads.  Lane l lands in row
   // l / CPR of its wave-load, physical chunk l % CPR, so it fetches the
   // logical chunk that the swizzle puts there.  Rows past M or N read a
-  // clamped valid row: they only feed outputs that are never stored.  The
+  // clamped valid row: they only feed outputs that are never stored.
   const std::uint16_t *src[LPW];
   int dst[LPW];
 #pragma unroll

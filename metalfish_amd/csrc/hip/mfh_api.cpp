@@ -109,6 +109,7 @@ constexpr int kSmolgenBiasRows = 48 * kSquares;
 // BF16X2_FP8LO: the fp8 lo correction runs from this many token rows (128
 // positions); below, the forward is the BF16X2 one.
 constexpr int kLo8MinRows = 8192;
+static_assert(kSmolgenBiasRows <= kLo8MinRows, "smolgen_bias.hip writes no e4m3 codes");
 // The body's residual LayerNorms are folded into the GEMMs around them
 // (GemmParams: the residual GEMMs write x o gamma with per-row partial sums,
 // Q|K|V, the compression and FFN1 take the LayerNorm in their epilogue, the
@@ -1076,15 +1077,15 @@ size_t PlanLayout(const Dims &d, int batch, size_t splitk_floats, bool side,
     add("hid8", M * (hid ? hid : 1));
     add("sc_hid", M * 4);
   }
-  // e4m3 lo parts of the encoder GEMM inputs (BF16X2_FP8LO), at the batches
-  // whose forward uses them.
   if (d.fold_ln && d.split && !d.fp8_act && !d.fused_ln &&
       d.E % (2 * mfh::kLnStatCols) == 0 && M >= static_cast<size_t>(kFoldRows)) {
     // Per-row partial sums of the folded LayerNorms' rows (LN2: "st_act",
-    // LN1: "st_mid"), per 64 columns at most.
-    add("st_act", M * (d.E / 64) * 2 * 4);
-    add("st_mid", M * (d.E / 64) * 2 * 4);
+    // LN1: "st_mid"), a pair per kLnStatCols columns.
+    add("st_act", M * (d.E / mfh::kLnStatCols) * 2 * 4);
+    add("st_mid", M * (d.E / mfh::kLnStatCols) * 2 * 4);
   }
+  // e4m3 lo parts of the encoder GEMM inputs (BF16X2_FP8LO), at the batches
+  // whose forward uses them.
   if (d.lo8 && M >= static_cast<size_t>(kLo8MinRows)) {
     add("act_lo8", M * d.E);
     add("qkv_lo8", M * 3 * d.E);
@@ -1605,8 +1606,9 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
   }
 
   // Dense2's LayerNorm and the global projection in one launch.
-  const bool smolgen_bias =
-      d.smolgen && !d.fused_bias && M < kSmolgenBiasRows && mfh::SmolgenBiasOk(d.H, d.G, kSquares * kSquares);
+  // (M below kLo8MinRows: no e4m3 codes of the bias.)
+  const bool smolgen_bias = d.smolgen && !d.fused_bias && M < kSmolgenBiasRows &&
+                            mfh::SmolgenBiasOk(d.H, d.G, kSquares * kSquares);
   // Single position (M <= 64 token rows, bf16 weights) where the shapes rule
   // that launch out (over 32 heads, another gen width): the smolgen chain
   // runs as three few-row GEMM launches instead of six (split-K GEMMs with
@@ -1630,7 +1632,7 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
                              mfh::SkinnyShapeOk(B, d.HG, d.Hs);
   auto run_bias = [&](const mfh::SmolgenBiasParams &p, hipStream_t s) {
     const double rows = static_cast<double>(p.batch) * p.heads;
-    const double out_bytes = p.out_lo8 ? 3.0 : p.split ? 4.0 : 2.0;
+    const double out_bytes = p.split ? 4.0 : 2.0;
     StageTimer t(net, s, "gemm_bf16:smolgen_global",
                  2.0 * rows * p.N * p.gen,
                  rows * (4.0 * p.gen + out_bytes * p.N) + (p.W8 ? 1.0 : 2.0) * p.N * p.gen);
@@ -1791,7 +1793,7 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
                              const size_t (&fc)[2], size_t skip) {
       p.ln_stats = st;
       p.ln_width = E;
-        p.ln_eps = eps;
+      p.ln_eps = eps;
       p.fold_c = net->W<float>(fc[0]) + skip;
       p.bias = net->W<float>(fc[1]) + skip;
     };
@@ -1807,7 +1809,8 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
     const bool chain_beside = side_chain && ws.Has("splitk_sg");
     hipStream_t sg_stream = chain_beside && !net->profiling ? net->side : st;
     mfh::GemmParams pq = gemm("act", E, L.qkv_w, E, M,
-                              3 * E + (L.smolgen && !side_chain ? d.C : 0), E, net->W<float>(L.qkv_b), mfh::ACT_NONE, mfh::GEMM_OUT_BF16,
+                              3 * E + (L.smolgen && !side_chain ? d.C : 0), E,
+                              net->W<float>(L.qkv_b), mfh::ACT_NONE, mfh::GEMM_OUT_BF16,
                               ws.S<std::uint16_t>("qkv"), ws.Lo("qkv"), 3 * E);
     if (L.smolgen && !side_chain) {
       pq.split_n = 3 * E;
@@ -1861,10 +1864,6 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
       // allow, else the LayerNorm, then the projection as a GEMM (unless
       // attention projects the gen vectors itself).
       auto smolgen_global = [&](hipStream_t s) -> int {
-        // BF16X2_FP8LO: the bias as bf16 hi plus the e4m3 codes of its lo
-        // parts (3 bytes instead of fp32's 4, written here and read by
-        // attention).
-        std::uint8_t *codes = qkv_codes ? ws.S<std::uint8_t>("bias_lo8") : nullptr;
         if (smolgen_bias) {
           mfh::SmolgenBiasParams pb;
           pb.x = sg2;
@@ -1882,7 +1881,6 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
           pb.N = kSquares * kSquares;
           pb.split = d.split_attn;
           pb.out = ws.S<void>("bias");
-          pb.out_lo8 = codes;
           MFH_RUN(run_bias(pb, s));
           return MFH_OK;
         }
@@ -1895,9 +1893,12 @@ int Forward(mfh_net *net, const WsView &ws, int B, const std::uint64_t *masks,
                                         kSquares * kSquares, d.G, nullptr,
                                         d.split_attn ? mfh::GEMM_OUT_F32 : mfh::GEMM_OUT_BF16,
                                         ws.S<void>("bias"), nullptr, kSquares * kSquares);
-        if (codes) {
+        if (qkv_codes) {
+          // BF16X2_FP8LO: the bias as bf16 hi plus the e4m3 codes of its lo
+          // parts (3 bytes instead of fp32's 4, written here and read by
+          // attention).
           pg.out_mode = mfh::GEMM_OUT_BF16;
-          pg.C_lo8 = codes;
+          pg.C_lo8 = ws.S<std::uint8_t>("bias_lo8");
           pg.ldc8 = kSquares * kSquares;
         }
         MFH_RUN(run(pg, "smolgen_global", s));

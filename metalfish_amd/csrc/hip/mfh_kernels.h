@@ -388,8 +388,7 @@ constexpr int SmolgenBiasIndex(int query, int key) {
 // launch: rows x [batch][heads * gen] fp32 (dense2's activated output),
 // out[batch * heads][N] = LN(x)[b][h segment] . W[N][gen]^T, the LayerNorm
 // over the whole heads * gen row.  `split`: the normalised rows as bf16 hi +
-// lo, fp32 output, or with out_lo8 bf16 plus e4m3 codes of the lo parts;
-// otherwise single bf16 rows and output.
+// lo, fp32 output; otherwise single bf16 rows and output.
 struct SmolgenBiasParams {
   const float *x = nullptr;
   const float *gamma = nullptr, *beta = nullptr;
@@ -401,7 +400,6 @@ struct SmolgenBiasParams {
   int N = 0;
   bool split = false;
   void *out = nullptr;
-  std::uint8_t *out_lo8 = nullptr;
   // Set by LaunchSmolgenBias: positions and column tiles per workgroup,
   // 16-bit reciprocal of a position's 256-element chunks.
   int positions = 0, tiles = 0, chunk_inv = 0;

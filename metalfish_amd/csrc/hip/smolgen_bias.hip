@@ -78,9 +78,8 @@ constexpr int Stages(int kb, bool split, bool w8) {
   return kFirst + (more < 3 ? more : 3);
 }
 
-// KB: gen width / 64.  OUT: 0 fp32, 1 bf16, 2 bf16 + e4m3
-// codes of the lo parts.
-template <int KB, bool SPLIT, int OUT, bool W8>
+// KB: gen width / 64.  SPLIT: bf16 hi + lo rows and fp32 output, else bf16.
+template <int KB, bool SPLIT, bool W8>
 __global__ __launch_bounds__(kWaves * 64, 2) void SmolgenBiasKernel(SmolgenBiasParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int P = SPLIT ? 2 : 1;
@@ -354,7 +353,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void SmolgenBiasKernel(SmolgenBiasP
         if constexpr (W8)
           o[r] *= sc[r];
       }
-      if constexpr (OUT == 0) {
+      if constexpr (SPLIT) {
         float *d = static_cast<float *>(p.out) + off;
         *reinterpret_cast<f32x4 *>(d) = f32x4{o[0], o[1], o[2], o[3]};
         *reinterpret_cast<f32x4 *>(d + 4) = f32x4{o[4], o[5], o[6], o[7]};
@@ -364,26 +363,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void SmolgenBiasKernel(SmolgenBiasP
         for (int r = 0; r < 4; ++r)
           h[r] = pack_bf16x2(o[2 * r], o[2 * r + 1]);
         *reinterpret_cast<u32x4 *>(static_cast<std::uint16_t *>(p.out) + off) = h;
-        if constexpr (OUT == 2) {
-          float l[8];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            l[2 * r] = o[2 * r] - __uint_as_float(h[r] << 16);
-            l[2 * r + 1] = o[2 * r + 1] - __uint_as_float(h[r] & 0xFFFF0000u);
-          }
-          *reinterpret_cast<u32x2 *>(p.out_lo8 + off) =
-              u32x2{Lo8Pack4(l[0], l[1], l[2], l[3]), Lo8Pack4(l[4], l[5], l[6], l[7])};
-        }
       }
     }
   }
 #endif
 }
 
-template <int KB, bool SPLIT, int OUT, bool W8>
+template <int KB, bool SPLIT, bool W8>
 hipError_t Launch(const SmolgenBiasParams &p, dim3 grid, hipStream_t stream) {
   constexpr int lds = kFirst * StageBytes(W8) + RowBytes(KB, SPLIT) + (W8 ? kMaxN * 4 : 0);
-  auto kernel = SmolgenBiasKernel<KB, SPLIT, OUT, W8>;
+  auto kernel = SmolgenBiasKernel<KB, SPLIT, W8>;
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [&]() {
@@ -396,17 +385,14 @@ hipError_t Launch(const SmolgenBiasParams &p, dim3 grid, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int KB, bool SPLIT, int OUT>
+template <int KB, bool SPLIT>
 hipError_t LaunchW(const SmolgenBiasParams &p, dim3 grid, hipStream_t stream) {
-  return p.W8 ? Launch<KB, SPLIT, OUT, true>(p, grid, stream)
-              : Launch<KB, SPLIT, OUT, false>(p, grid, stream);
+  return p.W8 ? Launch<KB, SPLIT, true>(p, grid, stream)
+              : Launch<KB, SPLIT, false>(p, grid, stream);
 }
 
 template <int KB> hipError_t LaunchK(const SmolgenBiasParams &p, dim3 grid, hipStream_t stream) {
-  if (p.out_lo8)
-    return LaunchW<KB, true, 2>(p, grid, stream);
-  return p.split ? LaunchW<KB, true, 0>(p, grid, stream)
-                 : LaunchW<KB, false, 1>(p, grid, stream);
+  return p.split ? LaunchW<KB, true>(p, grid, stream) : LaunchW<KB, false>(p, grid, stream);
 }
 
 bool Aligned16(const void *ptr) { return (reinterpret_cast<std::uintptr_t>(ptr) & 15) == 0; }
@@ -430,10 +416,10 @@ hipError_t LaunchSmolgenBias(const SmolgenBiasParams &p_in, hipStream_t stream,
     return fail("up to 32 heads, gen width 64, 128 or 256, heads x gen a multiple of 256, N a "
                 "multiple of 128 up to 4096");
   if (!p.x || !p.gamma || !p.beta || !p.out || (!p.W && !p.W8) || (p.W && p.W8) ||
-      (p.W8 && !p.wscale) || (p.out_lo8 && !p.split))
-    return fail("null operand (or both W and W8, or codes without split rows)");
+      (p.W8 && !p.wscale))
+    return fail("null operand (or both W and W8)");
   if (!Aligned16(p.x) || !Aligned16(p.gamma) || !Aligned16(p.beta) || !Aligned16(p.out) ||
-      !Aligned16(p.W) || !Aligned16(p.W8) || !Aligned16(p.wscale) || !Aligned16(p.out_lo8))
+      !Aligned16(p.W) || !Aligned16(p.W8) || !Aligned16(p.wscale))
     return fail("operands must be 16-byte aligned");
   // Whole positions per workgroup, and column tiles per workgroup such that
   // the rounds of 256 workgroups (one per CU) cost least: a tile takes about
