@@ -72,10 +72,10 @@ def test_row_quantisation_library_matches_numpy():
     assert np.allclose(deq3, deq, rtol=2 ** -22, atol=0)
 
 
-def _fp8_parity(spec_name, n, seed=0, batch=None, precision="bf16x2"):
+def _fp8_parity(spec_name, n, seed=0, batch=None, precision="bf16x2", fused_layernorm=False):
     """Parity of an fp8 net on n positions against the oracle; with `batch`,
-    the positions fill a batch of that size cyclically (large batches take
-    the row-panel GEMMs) and every copy is compared."""
+    the positions fill a batch of that size cyclically and every copy is
+    compared."""
     import oracle
 
     spec = synth.SPECS[spec_name]
@@ -85,7 +85,7 @@ def _fp8_parity(spec_name, n, seed=0, batch=None, precision="bf16x2"):
     batch = batch or n
     idx = np.arange(batch) % n
     net = backend.create_network(spec, weights, max_batch=batch, device=0, weights_dtype="fp8",
-                                 precision=precision)
+                                 precision=precision, fused_layernorm=fused_layernorm)
     gpu = net.evaluate_batch(planes[idx])
     net.close()
     planes, legal = planes[idx], legal[idx]
@@ -106,10 +106,21 @@ def _fp8_parity(spec_name, n, seed=0, batch=None, precision="bf16x2"):
 def test_fp8_weight_parity(spec_name, n, batch):
     """fp8-weight nets (bf16x2 activations) against the oracle running on the
     same dequantised weights; 40 BT4 positions reach the large-M tiles, a
-    batch of 128 the row-panel GEMMs with the fused LayerNorm."""
+    batch of 128 their 256-wide ones."""
     if backend.device_count() < 1:
         pytest.fail("GPU tests need an MI355X; none visible")
     perr, werr, agree = _fp8_parity(spec_name, n, batch=batch)
+    assert perr <= 1e-3 and werr <= 1e-4 and agree == 1.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spec_name,n", [("cpu_plumbing", 16), ("bt4", 40)])
+def test_fp8_weight_parity_row_panel(spec_name, n):
+    """The same at a batch of 128 with the row-panel GEMMs and their fused
+    LayerNorm (asked for, as only nets of width 256 take them by themselves)."""
+    if backend.device_count() < 1:
+        pytest.fail("GPU tests need an MI355X; none visible")
+    perr, werr, agree = _fp8_parity(spec_name, n, batch=128, fused_layernorm=True)
     assert perr <= 1e-3 and werr <= 1e-4 and agree == 1.0
 
 

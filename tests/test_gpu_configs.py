@@ -8,8 +8,7 @@
   against the CPU oracle on the same dequantised weights, and the four
   copies of each position agree bit for bit (each row's arithmetic does not
   depend on its slot).  At 65,536 token rows the Q|K|V and FFN1 GEMMs take
-  the whole-round 256 x 256 e4m3-weight tiles and the residual GEMMs the
-  row-panel kernel with the fused LayerNorm.
+  the whole-round 256 x 256 e4m3-weight tiles, as do the residual GEMMs.
 * Config 4: one encoder layer alone (``mfh_debug_encoder_layer``, the
   microbenchmark bench.py's ``encoder_layer`` line times) in single bf16 at
   batches 256 and 1024 on bf16 N(0, 1) inputs, checked stage by stage

@@ -151,14 +151,12 @@ def test_bt4_net_parity_16_positions(precision):
 @pytest.mark.parametrize("precision,n", [("bf16x2", 40), ("bf16", 40), ("bf16x2", 33),
                                          ("bf16x2", 28)])
 def test_bt4_large_batch_tiles(precision, n):
-    """40 positions = 2560 token rows: the dense layers take the large-M tile
-    configurations: 256 x 128 split tiles for Q|K|V (240 tiles; bf16: 128 x
-    128 / 256 x 128 ones), and the 64 x 64 tiles that split precision uses
-    below one 128 x 128 tile per CU for the out-projection, FFN1 and FFN2
-    (160 / 240 / 160 tiles).  33 positions = 2112 rows: the 256 x 128 split
-    tiles of Q|K|V end in a partial tile of 64 rows.  28 positions = 1792
-    rows: the large-M tiles below 2048 rows, with the smolgen chain on the
-    second stream."""
+    """40 positions = 2560 token rows: the dense layers take the large-M tiles,
+    Q|K|V the 128 x 256 ones beside the smolgen chain (240 tiles; bf16: 256 x
+    128), the out-projection, FFN1 and FFN2 those of the time model.  33
+    positions = 2112 rows: the tiles of Q|K|V end in a partial one of 64
+    rows.  28 positions = 1792 rows: the large-M tiles below 2048 rows, with
+    the smolgen chain on the second stream."""
     gpu, ref, legal = _compare("bt4", n, check_packed=False, precision=precision)
     perr = np.abs(gpu["policy"] - ref["policy"]).max()
     werr = np.abs(gpu["wdl"] - ref["wdl"]).max()
@@ -175,14 +173,13 @@ def test_bt4_large_batch_tiles(precision, n):
 @pytest.mark.parametrize("batch", [256, 512])
 def test_bt4_batch_256_whole_round_tiles(batch):
     """Batch 256 (16384 token rows, the benchmark batch): the dense layers
-    whose tile count fills whole rounds of 256 workgroups (out-projection,
-    FFN2, smolgen global) take the 256 x 256 eight-wave tiles, which no
-    smaller batch reaches, and the body's residual LayerNorms are folded
-    into the GEMMs around them; at batch 512 FFN1 takes whole-round 256 x
-    256 tiles too.  The 40 oracle-checked positions fill the batch
-    cyclically; each copy meets the bf16x2 gates against the oracle and agrees
-    with the batch-40 run (other tile shapes, no fold) to summation-order
-    noise."""
+    whose tile count fills whole rounds of 256 workgroups (Q|K|V,
+    out-projection, FFN2) take the 256 x 256 eight-wave tiles, and the body's
+    residual LayerNorms are folded into the GEMMs around them; at batch 512
+    FFN1 takes whole-round 256 x 256 tiles too.  The 40 oracle-checked
+    positions fill the batch cyclically; each copy meets the bf16x2 gates
+    against the oracle and agrees with the batch-40 run (other tile shapes) to
+    summation-order noise."""
     spec = synth.SPECS["bt4"]
     weights, planes, legal, ref = _reference("bt4", 40, 0, 0)
     idx = np.arange(batch) % 40
@@ -213,8 +210,7 @@ def test_folded_layernorm_row_widths(embedding, heads, ffn, gen, batches):
     per-row partial sums, each row's four-lane group one lane short) and
     2048 (eight quads: the load rounds past the two prefetched ones run in
     the staging), two layers with smolgen (the compression GEMM takes the
-    folded rows too); FFN1 takes 256 x 256 tiles at 768 and 256 x 128 tiles
-    at 2048.  Batch 255 folds with a partial last row tile; batches 1000
+    folded rows too).  Batch 255 folds with a partial last row tile; batches 1000
     and 252 are no whole rounds and keep the LayerNorm kernels: the folded
     forwards run 2L - 1 = 3 fewer LayerNorm launches than those.  Every
     position meets the gates against the oracle, and the folded and
@@ -278,11 +274,11 @@ def test_folded_layernorm_switch(monkeypatch):
 @pytest.mark.parametrize("batch", [24, 32])
 def test_folded_layernorms_small_batch(batch, monkeypatch):
     """From 24 positions, below whole rounds, both residual LayerNorms are
-    folded on the 64 x 64 residual tiles (partial sums per 64 columns): the
+    folded (partial sums per 128 columns): the
     out-projection writes x o gamma1, FFN1 applies LN1 in its epilogue and
     FFN2 rebuilds its residual from it; FFN2 writes x o gamma2, the next
-    layer's Q|K|V (256 x 128 tiles) applies LN2 in its epilogue, the
-    smolgen compression (split over K) in its reduce kernel, and the next
+    layer's Q|K|V applies LN2 in its epilogue, the smolgen compression (narrow
+    tiles, K over the waves) in its own, and the next
     out-projection rebuilds its residual.  2L - 1 = 3 LayerNorm launches
     fewer than with METALFISH_HIP_FOLD_LN=0 (the last layer's LN2 feeds the
     heads), the same outputs to summation-order noise, and the gates against
@@ -317,11 +313,9 @@ def test_folded_layernorms_small_batch(batch, monkeypatch):
 
 @pytest.mark.parametrize("batch", [48, 56])
 def test_bt4_folded_layernorms_wide_ffn1(batch, monkeypatch):
-    """43-62 positions at the BT4 widths: the residual GEMMs still take 64 x
-    64 tiles (fewer than 256 128 x 128 tiles), FFN1 (N = 1536) takes 128 x
-    128 tiles without the fold, and both LayerNorms stay folded, FFN1
-    applying LN1 on up to two rounds of 64 x 64 tiles (partial sums per 64
-    columns).  The 40 oracle-checked positions
+    """43-62 positions at the BT4 widths, where the residual GEMMs have
+    fewer than 256 tiles of 128 x 128 and FFN1 (N = 1536) more: both
+    LayerNorms are folded.  The 40 oracle-checked positions
     fill the batch cyclically; each copy meets the bf16x2 gates, the forward
     agrees with the unfolded one (METALFISH_HIP_FOLD_LN=0) to
     summation-order noise, and it makes 2L - 1 LayerNorm launches fewer."""
@@ -455,12 +449,13 @@ def test_bt4_small_batch_parity(batch):
     ("bt4", "bf16x2"), ("bt4", "bf16x2_gemm"), ("bt4", "bf16"),
     ("cpu_plumbing_smolgen", "bf16x2"), ("cpu_plumbing_smolgen", "bf16")])
 def test_single_position_few_row_path(spec_name, precision, monkeypatch):
-    """At batch 1 the smolgen chain runs as three few-row GEMM launches, each
-    of its LayerNorms applied by the GEMM that reads its output (the global
-    projection normalises each position's whole gen row and reads one head's
-    segment).  Position by position against the oracle, and against the
-    split-K chain with separate LayerNorm launches (METALFISH_HIP_SKINNY=0):
-    the two differ only in fp32 summation order."""
+    """At batch 1 the smolgen chain's dense layers run as few-row GEMM
+    launches, dense2 applying dense1's LayerNorm as it loads its rows; dense2's
+    LayerNorm and the global projection follow in one launch.  Position by
+    position against the oracle, and against the split-K dense layers with
+    a LayerNorm launch between them (METALFISH_HIP_SKINNY=0): the two differ
+    only in fp32 summation order.  (Shapes that the one launch does not take:
+    test_gpu_smolgen_bias.py.)"""
     spec = synth.SPECS[spec_name]
     seed = 0 if spec_name == "bt4" else 7
     weights, planes, legal, ref = _reference(spec_name, 16, seed, 0)

@@ -7,6 +7,7 @@ import dataclasses
 import numpy as np
 import pytest
 
+import oracle
 from metalfish_amd import backend, synth
 
 pytestmark = pytest.mark.gpu
@@ -46,3 +47,46 @@ def test_bias_agrees_with_attention_kernel(heads, gen, precision, weights_dtype,
         assert err <= tol
     net.close()
     ref.close()
+
+
+@pytest.mark.parametrize("heads,gen", [(40, 64), (8, 192)])
+@pytest.mark.parametrize("precision", ["bf16x2", "bf16x2_gemm", "bf16"])
+def test_shapes_without_the_one_launch(heads, gen, precision, monkeypatch):
+    """More than 32 heads, or a gen width other than 64, 128 and 256: at one
+    position the chain is three few-row launches, each LayerNorm applied by
+    the GEMM that reads its rows (2L LayerNorm launches fewer than the split-K
+    chain, METALFISH_HIP_SKINNY=0); at two, dense1's LayerNorm alone (L
+    fewer), then dense2's and the projection GEMM; at 24, all separate.
+    Against the oracle and that chain, with the bounds of those precisions
+    (bf16x2: summation order, 1e-4; the others round activations to bf16)."""
+    layers = 2
+    spec = dataclasses.replace(synth.SPECS["bt4"], name="other", layers=layers,
+                               embedding=heads * 32, heads=heads, ffn=512, input_ffn=512,
+                               smolgen_gen=gen, smolgen_hidden=64, smolgen_compress=8,
+                               policy_dim=256)
+    weights = synth.make_weights(spec, seed=8)
+    planes, _ = synth.playout_positions(4, seed=8)
+    ref = oracle.OracleNet(oracle.NetFormat(body_heads=heads), weights).evaluate_batch(planes)
+    outs, lns = {}, {}
+    for skinny in ("1", "0"):
+        monkeypatch.setenv("METALFISH_HIP_SKINNY", skinny)
+        net = backend.create_network(spec, weights, max_batch=24, device=0, precision=precision)
+        net.set_profiling(True)
+        for batch in (1, 2, 24):
+            net.profile_reset()
+            outs[skinny, batch] = net.evaluate_batch(planes[np.arange(batch) % 4])
+            lns[skinny, batch] = net.profile()["layernorm"]["launches"]
+        net.close()
+    ptol, wtol, dtol = {"bf16x2": (1e-3, 1e-4, 1e-4), "bf16x2_gemm": (2e-2, 5e-3, 2e-2),
+                        "bf16": (3e-2, 5e-3, 2e-2)}[precision]
+    for (skinny, batch), out in outs.items():
+        idx = np.arange(batch) % 4
+        perr = np.abs(out["policy"] - ref["policy"][idx]).max()
+        werr = np.abs(out["wdl"] - ref["wdl"][idx]).max()
+        diff = np.abs(out["policy"] - outs["0", batch]["policy"]).max()
+        print(f"{heads} x {gen} {precision} batch {batch} skinny {skinny}: policy {perr:.2e} "
+              f"wdl {werr:.2e}, from the split-K chain {diff:.2e}, "
+              f"{lns[skinny, batch]} LayerNorms", flush=True)
+        assert perr <= ptol and werr <= wtol and diff <= dtol
+    for batch, fewer in ((1, 2 * layers), (2, layers), (24, 0)):
+        assert lns["1", batch] == lns["0", batch] - fewer, batch

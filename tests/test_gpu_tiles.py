@@ -1,7 +1,8 @@
-"""The GEMM tiles of the larger shapes (from 256 rows): every tile gives the
-bits of the 64 x 64 tiles that small shapes take, and forwards at batches
-where the choice of tile, a row split or the LayerNorm fold changes agree
-with small batches."""
+"""The GEMM tiles of the larger shapes (from 256 rows): the single-bf16 tiles
+give the bits of the 64 x 64 ones that small shapes take, forwards of every
+precision give a position the same bits on all tiles that a batch may take,
+and forwards at batches where the choice of tile, a row split or the LayerNorm
+fold changes agree with small batches."""
 
 import dataclasses
 
@@ -29,9 +30,9 @@ def _bits(rng, shape, scale=1.0):
                                    (700, 1538, 512), (1030, 3136, 1024), (1535, 1536, 640)])
 @pytest.mark.parametrize("act", ["none", "mish"])
 def test_large_tiles_equal_small_ones(m, n, k, act):
-    """The MFMAs of an output accumulate over K in one order on every tile,
-    so a row's bits do not depend on how many rows the call has (the small
-    call's 64 x 64 tiles run over the whole K); float64 bounds the product:
+    """Single bf16 with fp32 output: the MFMAs of an output accumulate over
+    K in one order on every tile, so a row's bits do not depend on how many
+    rows the call has (the small call's 64 x 64 tiles run over the whole K); float64 bounds the product:
     at most K * 2^-24 of the summed magnitudes, with a factor 2 for the
     products' own rounding, and mish's slope is below 1.1."""
     rng = np.random.default_rng(m * 7 + n + k)
@@ -94,6 +95,61 @@ def test_lo8_rows_past_2_gib():
     small = backend.gemm_lo8(a[rows], a8[rows], w, w8, scale, bf16_out=True)
     for got, want in zip(out, small):
         assert np.array_equal(got[rows], want)
+
+
+# Batches of one group take different tiles, row splits and edges, but the same
+# K order everywhere else (below 24 some products are split over K; the policy
+# map and the smolgen compression change theirs at 65, the compression at 48).
+_BIT_GROUPS = {
+    ("plain", "0"): [[24, 25, 33, 43, 48, 63, 64], [65, 86, 100, 129, 200, 255, 256, 257, 300, 321,
+                                                    513]],
+    ("smolgen", "0"): [[48, 62, 63, 64], [65, 66, 86, 100, 129, 200, 255, 256, 257, 300, 321, 513]],
+    ("plain", "1"): [[24, 25, 33, 43, 48, 62], [63, 64], [65, 100, 257, 300], [255, 256, 512]],
+    ("smolgen", "1"): [[48, 62], [255, 256, 512]],
+}
+# K of one, two, three and eight 64-wide stages: fewer, as many and more than a
+# ring holds.  (No e4m3 net of width 256, which takes the row panel at 128.)
+_BIT_GROUPS["narrow", "0"] = _BIT_GROUPS["middle", "0"] = _BIT_GROUPS["plain", "0"]
+_BIT_KINDS = {
+    "smolgen": {},
+    "plain": dict(smolgen_compress=0, smolgen_hidden=0, smolgen_gen=0),
+    "narrow": dict(smolgen_compress=0, smolgen_hidden=0, smolgen_gen=0, embedding=128, heads=4,
+                   ffn=64, input_ffn=64, policy_dim=128),
+    "middle": dict(smolgen_compress=0, smolgen_hidden=0, smolgen_gen=0, embedding=512, heads=16,
+                   ffn=192, input_ffn=192, policy_dim=64),
+}
+
+
+@pytest.mark.parametrize("kind,precision,weights_dtype,fold", [
+    (kind, precision, dtype, fold) for kind, fold in _BIT_GROUPS for precision, dtype in (
+        ("bf16x2", "bf16"), ("bf16x2_gemm", "bf16"), ("bf16x2", "fp8"), ("bf16", "bf16"),
+        ("bf16", "fp8")) if fold == "0" or (precision != "bf16" and dtype == "bf16")])
+def test_a_position_has_the_same_bits_on_every_tile(kind, precision, weights_dtype, fold,
+                                                    monkeypatch):
+    """Two layers of the BT4 width and narrower, the split, e4m3, residual and
+    folded epilogues and the row splits among them: each position of a batch
+    has the bits that the other batches of its group give it."""
+    monkeypatch.setenv("METALFISH_HIP_FOLD_LN", fold)
+    spec = dataclasses.replace(synth.SPECS["bt4"], name="bits", layers=2, **_BIT_KINDS[kind])
+    weights = synth.make_weights(spec, seed=3)
+    planes, _ = synth.playout_positions(8, seed=4)
+    net = backend.create_network(spec, weights, max_batch=513, device=0, precision=precision,
+                                 weights_dtype=weights_dtype)
+    for group in _BIT_GROUPS[kind, fold]:
+        want = None
+        for batch in group:
+            idx = (np.arange(batch) * 5 + batch) % 8
+            out = net.evaluate_batch(planes[idx])
+            got = {k: np.ascontiguousarray(out[k]).view(np.uint32) for k in ("policy", "wdl")}
+            if want is None:
+                want = {k: np.stack([got[k][np.flatnonzero(idx == i)[0]] for i in range(8)])
+                        for k in got}
+            for k in got:
+                bad = np.flatnonzero((got[k] != want[k][idx]).any(axis=1))
+                print(f"{kind} {precision}/{weights_dtype} fold {fold} batch {batch} {k}: "
+                      f"{bad.size} positions differ", flush=True)
+                assert bad.size == 0, (batch, k, bad[:8])
+    net.close()
 
 
 @pytest.mark.parametrize("weights_dtype", ["bf16", "fp8"])
