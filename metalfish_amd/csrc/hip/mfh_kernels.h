@@ -120,8 +120,8 @@ struct GemmParams {
   //   out = act(r (acc - mu fold_c[n]) + bias[n]) with the stats ln_stats;
   // * residual y (res_stats set): resid16 / resid16_lo hold x o gamma, and
   //   resid = r (x o gamma - mu res_gamma) + res_beta.
-  // Residual modes with out_gamma or res_stats take whole tiles of 256 or
-  // 128 columns (LaunchGemm rejects other shapes).
+  // bf16 weights only; residual modes with out_gamma or res_stats take whole
+  // tiles of 256 or 128 columns (LaunchGemm rejects others).
   const float *ln_stats = nullptr;
   const float *fold_c = nullptr;
   float ln_eps = 0.f;
