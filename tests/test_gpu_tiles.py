@@ -97,6 +97,27 @@ def test_lo8_rows_past_2_gib():
         assert np.array_equal(got[rows], want)
 
 
+@pytest.mark.parametrize("precision,weights_dtype", [("bf16x2", "bf16"), ("bf16x2", "fp8"),
+                                                     ("bf16", "bf16")])
+def test_net_with_hidden_rows_past_2_gib(precision, weights_dtype):
+    """4200 positions with an FFN of width 4096: FFN2 reads 2.2 GB of hidden
+    rows (each plane), with the residual; every position has the bits of
+    batch 321."""
+    spec = dataclasses.replace(synth.SPECS["bt4"], name="wide", layers=1, ffn=4096)
+    weights = synth.make_weights(spec, seed=1)
+    planes, _ = synth.playout_positions(8, seed=2)
+    masks, values = backend.pack_planes(planes)
+    net = backend.create_network(spec, weights, max_batch=4200, device=0, precision=precision,
+                                 weights_dtype=weights_dtype)
+    idx = np.arange(4200) % 8
+    policy, wdl = net.eval_packed(masks[idx], values[idx])
+    small_policy, small_wdl = net.eval_packed(masks[idx[:321]], values[idx[:321]])
+    net.close()
+    assert np.isfinite(policy).all() and np.ptp(policy) > 0
+    assert np.array_equal(policy, small_policy[:8][idx])
+    assert np.array_equal(wdl, small_wdl[:8][idx])
+
+
 # Batches of one group take different tiles, row splits and edges, but the same
 # K order everywhere else (below 24 some products are split over K; the policy
 # map and the smolgen compression change theirs at 65, the compression at 48).
